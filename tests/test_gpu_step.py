@@ -404,3 +404,16 @@ def test_recycled_slot_starts_clean_after_async_step(gpu, orc):
         assert not np.any(k) and not np.any(v) and not np.any(c), "layer %d" % l
     enc.close()
 
+
+
+@pytest.mark.parametrize("S,T", [(129, 1), (13, 11), (107, 3), (64, 11), (161, 7), (163, 11), (200, 14)])
+def test_step_bf16_projection_tiles(gpu, orc, S, T):
+    """129 to 2,800 rows in one layer: each kernel that the 16-bit projections choose between (64 x 64
+    and 64 x 32 register tiles, 64 x 128, 128 x 128 and 112 x 256 row panels, one or several K splits), at row
+    counts that leave a ragged last tile; some chunks partly valid."""
+    cfg = gpu.EncoderConfig(layers=1, max_chunk=T, max_streams=S, dtype="bf16")
+    plan = lambda step, S, T: [T - (s % 4 == 1) * min(T, 1 + s % 3) for s in range(S)]
+    enc, _, _, res = _run_steps(gpu, orc, cfg, S=S, T=T, n_steps=1, seed=61 + S, seed_caches=True, valid_plan=plan)
+    for got, ref in res:
+        harness.assert_bf16_close(got, ref, "%d x %d" % (S, T))
+    enc.close()

@@ -812,7 +812,7 @@ static int enqueue_rows(ud_encoder* e, int s0, int n, int T, const float* x, flo
                     const char* what) -> int {
         GemmArgs g{};
         g.A = A; g.W = W; g.C = C; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = ldc;
-        g.epi = epi; g.act = act; g.out_scale = scale; g.ksplit = 1; g.f16 = bf ? 1 : 0;
+        g.epi = epi; g.act = act; g.out_scale = scale; g.ksplit = 1;
         return launch_status(launch_gemm(g, bf, st), what);
     };
     // res += scale * A . W^T (N = D)
@@ -820,8 +820,8 @@ static int enqueue_rows(ud_encoder* e, int s0, int n, int T, const float* x, flo
         if (!bf) return gemm(A, W, w.res, D, K, D, EPI_RESID, ACT_NONE, scale, what);
         GemmArgs g{};
         g.A = A; g.W = W; g.C = w.part; g.M = M; g.N = D; g.K = K; g.lda = K; g.ldw = K; g.ldc = D;
-        g.epi = EPI_PARTIAL; g.act = ACT_NONE; g.out_scale = scale; g.f16 = 1;
-        g.ksplit = gemm_partial_splits(M, D, K, bf);
+        g.epi = EPI_PARTIAL; g.act = ACT_NONE; g.out_scale = scale;
+        g.ksplit = gemm_partial_splits(M, D, K);
         pend.n = g.ksplit;
         return launch_status(launch_gemm(g, bf, st), what);
     };
@@ -856,7 +856,7 @@ static int enqueue_rows(ud_encoder* e, int s0, int n, int T, const float* x, flo
             // q into the qkv buffer, the new K/V rows straight into the rings
             GemmArgs g{};
             g.A = w.z; g.W = l.wqkv; g.C = w.qkv; g.M = M; g.N = 3 * D; g.K = D; g.lda = D; g.ldw = D; g.ldc = 3 * D;
-            g.epi = EPI_QKV_RING; g.act = ACT_NONE; g.out_scale = 1.0f; g.ksplit = 1; g.f16 = 1;
+            g.epi = EPI_QKV_RING; g.act = ACT_NONE; g.out_scale = 1.0f; g.ksplit = 1;
             g.ring = QkvRing{ra.kring, ra.vring, w.rows, T, e->L, e->R, e->H};
             if ((rc = launch_status(launch_gemm(g, true, st), "qkv"))) return rc;
         } else {
@@ -1027,7 +1027,6 @@ extern "C" UD_API int ud_encoder_subsample(ud_encoder* e, int32_t n, int32_t mel
         GemmArgs g{};
         g.A = A; g.W = u.w[slot_w]; g.C = C; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
         g.epi = EPI_STORE_F32; g.act = act; g.out_scale = 1.0f; g.ksplit = 1; g.bias = (const float*)u.w[slot_b];
-        g.f16 = bf ? 1 : 0;
         return launch_status(launch_gemm(g, bf, st), what);
     };
     // conv.3: half channel-last rows for a 16-bit encoder (the depthwise conv.5 reads them), fp32 otherwise
@@ -1035,7 +1034,7 @@ extern "C" UD_API int ud_encoder_subsample(ud_encoder* e, int32_t n, int32_t mel
         GemmArgs g{};
         g.A = u.a2; g.W = u.w[SUB_C3W]; g.C = u.a3; g.M = n * T2 * SUB_F2; g.N = SUB_CH; g.K = SUB_CH;
         g.lda = SUB_CH; g.ldw = SUB_CH; g.ldc = SUB_CH; g.epi = bf ? EPI_STORE : EPI_STORE_F32; g.act = ACT_RELU;
-        g.out_scale = 1.0f; g.ksplit = 1; g.bias = (const float*)u.w[SUB_C3B]; g.f16 = bf ? 1 : 0;
+        g.out_scale = 1.0f; g.ksplit = 1; g.bias = (const float*)u.w[SUB_C3B];
         if ((rc = launch_status(launch_gemm(g, bf, st), "subsampling conv.3"))) return rc;
     }
     SubDwArgs dw{};
@@ -1047,7 +1046,7 @@ extern "C" UD_API int ud_encoder_subsample(ud_encoder* e, int32_t n, int32_t mel
         GemmArgs g{};
         g.A = u.a4; g.W = u.w[SUB_C6W]; g.C = u.af; g.M = n * T3 * SUB_F3; g.N = SUB_CH; g.K = SUB_CH;
         g.lda = SUB_CH; g.ldw = SUB_CH; g.ldc = SUB_CH; g.epi = EPI_SUBFLAT; g.act = ACT_RELU; g.out_scale = 1.0f;
-        g.ksplit = 1; g.bias = (const float*)u.w[SUB_C6B]; g.f16 = 1;
+        g.ksplit = 1; g.bias = (const float*)u.w[SUB_C6B];
         g.flat = SubFlat{u.vlen, T3, SUB_F3, T, drop};
         if ((rc = launch_status(launch_gemm(g, true, st), "subsampling conv.6 + flatten"))) return rc;
     } else {
@@ -1153,7 +1152,7 @@ static int launch_projection(ud_encoder* e, int which, int layer, int M, hipStre
     const int D = e->D, ff = e->ff;
     const LayerDev& l = e->lw[layer];
     GemmArgs g{};
-    g.M = M; g.ksplit = 1; g.out_scale = 1.0f; g.act = ACT_NONE; g.f16 = e->bf ? 1 : 0;
+    g.M = M; g.ksplit = 1; g.out_scale = 1.0f; g.act = ACT_NONE;
     switch (which) {
         case UD_PROJ_FF_LINEAR1:
             g.A = e->z; g.W = l.ff1_w1; g.C = e->h; g.N = ff; g.K = D; g.ldc = ff; g.act = ACT_SILU;
@@ -1183,7 +1182,7 @@ static int launch_projection(ud_encoder* e, int which, int layer, int M, hipStre
     }
     if (g.N == D) {                       // the residual projections: split-K slabs (16-bit) or +=
         g.ldc = D;
-        if (e->bf) { g.C = e->part; g.epi = EPI_PARTIAL; g.ksplit = gemm_partial_splits(M, D, g.K, true); }
+        if (e->bf) { g.C = e->part; g.epi = EPI_PARTIAL; g.ksplit = gemm_partial_splits(M, D, g.K); }
         else { g.C = e->res; g.epi = EPI_RESID; }
     }
     g.lda = g.K; g.ldw = g.K;

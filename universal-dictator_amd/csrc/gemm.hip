@@ -2,22 +2,27 @@
 // orientation (Sources/DictatorEngine/Core/Kernels.swift:79-112; epilogue order of
 // Sources/DictatorEngine/Metal/12_gemm2.metal:111-122: act, then out_scale, then + residual).
 //
-// bf16 path: v_mfma_f32_16x16x32_bf16 (gfx950).  The streaming step multiplies M = streams x T
-// rows (128 at 64 streams x 2 frames) against 2-8 MB weight matrices.  Measured on MI355X, the
-// limit at this shape is not HBM but the L2 -> CU traffic of the activation fragments, which every
-// column tile re-reads; so both operands are stored fragment-major (see frag_index): each operand
-// fragment is one contiguous 1 KB load, with no partially used cache lines.
-//  - each wave owns a [16*MT x 16*NT] output tile (shapes per GEMM in launch_bf16)
-//    and every WK-th 64-wide K chunk of its workgroup's K range; the WK waves are summed in LDS;
-//  - two register buffers, separated by scheduling barriers, keep the next chunk's loads in flight
-//    behind the current chunk's MFMAs;
+// 16-bit path: v_mfma_f32_16x16x32_f16 (gfx950) on IEEE-half operands.  The streaming step multiplies
+// M = streams x T rows (128 at 64 streams x 2 frames) against 2-8 MB weight matrices.  Measured on
+// MI355X, the limit at few rows is not HBM but the L2 -> CU traffic of the activation fragments, which
+// every column tile re-reads; so both operands are stored fragment-major (see frag_index): each
+// operand fragment is one contiguous 1 KB load, with no partially used cache lines.
+//  - gemm_bf16_kernel, few rows: each wave owns a [16*MT x 16*NT] output tile (shapes per GEMM in
+//    launch_few) and every WK-th 64-wide K chunk of its workgroup's K range; the WK waves are summed
+//    in LDS; two register buffers, separated by scheduling barriers, keep the next chunk's loads in
+//    flight behind the current chunk's MFMAs;
+//  - gemm_panel_kernel, many rows: the waves of a workgroup share a row panel through LDS and each
+//    stream their own weights;
+//  - plan16 chooses between them;
 //  - ksplit > 1 splits K over workgroups (parallelism for the N = 1024 projections); each split
 //    writes its own fp32 partial slab and the following LayerNorm adds the slabs, in order, to the
 //    residual row it reads anyway -- deterministic, no atomics, no extra kernel.
-// Epilogues: act + bf16 store (row-major, or fragment-major for a following GEMM), fp32 store,
+// Epilogues: act + half store (row-major, or fragment-major for a following GEMM), fp32 store,
 // in-place fp32 residual accumulate, split-K partial slabs, and the QKV projection's split store:
 // q row-major into the buffer the attention reads, K and V straight into their K/V ring rows (so
 // the new rows are written once, and the attention kernel only reads the rings).
+#include <type_traits>
+
 #include "ud_common.hpp"
 #include "kernels.hpp"
 
@@ -58,6 +63,11 @@ __device__ __forceinline__ int64_t subflat_dst(const GemmArgs& a, int64_t m, int
     return frag_index((int64_t)s * f.T + t3 - f.drop, f3 * a.N + n, f.F3 * a.N / 64);
 }
 
+// Four floats as IEEE half, packed.
+__device__ __forceinline__ uint2 pack4(float x, float y, float z, float w) {
+    return make_uint2((uint32_t)f2h(x) | ((uint32_t)f2h(y) << 16), (uint32_t)f2h(z) | ((uint32_t)f2h(w) << 16));
+}
+
 template <int MT, int NT>
 struct Frag {
     uint4 a[MT][2];
@@ -78,21 +88,16 @@ __device__ __forceinline__ void load_frag(Frag<MT, NT>& f, const bf16* const* ap
     }
 }
 
-template <int MT, int NT, bool H>
+template <int MT, int NT>
 __device__ __forceinline__ void mma_frag(const Frag<MT, NT>& f, f32x4_t (&acc)[NT][MT]) {
 #pragma unroll
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                if constexpr (H)
-                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_f16x8(f.a[mt][h]), as_f16x8(f.b[nt][h]),
-                                                                         acc[nt][mt], 0, 0, 0);
-                else
-                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f.a[mt][h]), as_bf16x8(f.b[nt][h]),
-                                                                          acc[nt][mt], 0, 0, 0);
-            }
+            for (int mt = 0; mt < MT; mt++)
+                acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_f16x8(f.a[mt][h]), as_f16x8(f.b[nt][h]),
+                                                                     acc[nt][mt], 0, 0, 0);
 }
 
 // Grid: (N/16) x ceil(M/(16*MT)) x ksplit workgroups of WK waves.  The host guarantees
@@ -100,7 +105,7 @@ __device__ __forceinline__ void mma_frag(const Frag<MT, NT>& f, f32x4_t (&acc)[N
 // .. of its split, so when WK does not divide the chunk count the first waves take one more.  The epilogue kind and activation are template parameters: a
 // runtime-switched, fully unrolled epilogue measured ~3.5 us slower per launch on MI355X (its
 // code does not stay in the instruction cache).
-template <int MT, int WK, int EPI, int ACT, int NT, bool H = false, bool BIAS = false>
+template <int MT, int WK, int EPI, int ACT, int NT, bool BIAS = false>
 __global__ __launch_bounds__(64 * WK, 1) void gemm_bf16_kernel(GemmArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -148,21 +153,21 @@ __global__ __launch_bounds__(64 * WK, 1) void gemm_bf16_kernel(GemmArgs a) {
     for (; i + 2 < cnt; i += 2) {
         load_frag(f1, ap, wp, off(i + 1));
         __builtin_amdgcn_sched_barrier(0);
-        mma_frag<MT, NT, H>(f0, acc);
+        mma_frag<MT, NT>(f0, acc);
         __builtin_amdgcn_sched_barrier(0);
         load_frag(f0, ap, wp, off(i + 2));
         __builtin_amdgcn_sched_barrier(0);
-        mma_frag<MT, NT, H>(f1, acc);
+        mma_frag<MT, NT>(f1, acc);
         __builtin_amdgcn_sched_barrier(0);
     }
     if (i + 1 < cnt) {
         load_frag(f1, ap, wp, off(i + 1));
         __builtin_amdgcn_sched_barrier(0);
-        mma_frag<MT, NT, H>(f0, acc);
+        mma_frag<MT, NT>(f0, acc);
         __builtin_amdgcn_sched_barrier(0);
-        mma_frag<MT, NT, H>(f1, acc);
+        mma_frag<MT, NT>(f1, acc);
     } else {
-        mma_frag<MT, NT, H>(f0, acc);
+        mma_frag<MT, NT>(f0, acc);
     }
 
     // Epilogue of one finished 16 x 16 accumulator (j, mt): the lane holds rows
@@ -180,17 +185,17 @@ __global__ __launch_bounds__(64 * WK, 1) void gemm_bf16_kernel(GemmArgs a) {
             } else if constexpr (EPI == EPI_STORE_F32) {
                 static_cast<float*>(a.C)[m * a.ldc + n] = apply_act(v, ACT) * a.out_scale;
             } else if constexpr (EPI == EPI_STORE_FRAG) {
-                static_cast<uint16_t*>(a.C)[frag_index(m, n, a.N / 64)] = to16<H>(apply_act(v, ACT) * a.out_scale);
+                static_cast<uint16_t*>(a.C)[frag_index(m, n, a.N / 64)] = f2h(apply_act(v, ACT) * a.out_scale);
             } else if constexpr (EPI == EPI_QKV_RING) {
-                const uint16_t x = to16<H>(apply_act(v, ACT) * a.out_scale);
+                const uint16_t x = f2h(apply_act(v, ACT) * a.out_scale);
                 if (n < a.ring.H * 128) static_cast<uint16_t*>(a.C)[m * a.ldc + n] = x;
                 else *qkv_ring_dst(a.ring, rtab[mt * 16 + g * 4 + i2], n) = x;
             } else if constexpr (EPI == EPI_SUBFLAT) {
                 bool masked;
                 const int64_t d = subflat_dst(a, m, n, masked);
-                if (d >= 0) static_cast<uint16_t*>(a.C)[d] = masked ? (uint16_t)0 : to16<H>(apply_act(v, ACT) * a.out_scale);
+                if (d >= 0) static_cast<uint16_t*>(a.C)[d] = masked ? (uint16_t)0 : f2h(apply_act(v, ACT) * a.out_scale);
             } else {
-                static_cast<uint16_t*>(a.C)[m * a.ldc + n] = to16<H>(apply_act(v, ACT) * a.out_scale);
+                static_cast<uint16_t*>(a.C)[m * a.ldc + n] = f2h(apply_act(v, ACT) * a.out_scale);
             }
         }
     };
@@ -202,7 +207,7 @@ __global__ __launch_bounds__(64 * WK, 1) void gemm_bf16_kernel(GemmArgs a) {
         for (int i2 = 0; i2 < 4; i2++) {
             const int64_t m = (int64_t)(mb * MT + mt) * 16 + g * 4 + i2;
             if (m >= a.M) continue;
-            static_cast<uint16_t*>(a.C)[m * a.ldc + c] = to16<H>(vv[i2] * sigmoidf(vg[i2]));
+            static_cast<uint16_t*>(a.C)[m * a.ldc + c] = f2h(vv[i2] * sigmoidf(vg[i2]));
         }
     };
     if constexpr (EPI == EPI_GLU) {
@@ -260,35 +265,48 @@ __global__ __launch_bounds__(64 * WK, 1) void gemm_bf16_kernel(GemmArgs a) {
     }
 }
 
-// ---------------------------------------------------------------- bf16, many rows (LDS-staged)
-// For M in the thousands (256 streams x 14 frames = 3584 rows) the projections are MFMA-bound, and
-// the register-direct kernel above would re-read each activation fragment once per 16-column tile.
-// Here a workgroup of 8 waves (2 per SIMD, so one wave's MFMAs run while the other waits on LDS)
-// owns a 256 x 64*NT output tile (or 224 or 128 rows).  Per 32-deep K step it copies the row
-// fragments and 4*NT column fragments (each a contiguous 1 KB half of a 2 KB fragment-major block,
-// so the copy is linear) into LDS with direct global -> LDS loads (global_load_lds_dwordx4, no
-// staging registers).  LDS holds a ring of four steps and the fragments are read one step ahead:
-// at step s the wave waits until its own loads of step s+1 have landed (those of s+2 and s+3 may
-// still be in flight) and its LDS reads of step s are done, a barrier makes every wave's loads
-// visible and frees step s's buffer, the wave reads its step-(s+1) fragments into its second
-// register set, issues the loads of step s+4 into step s's buffer, and multiplies step s.  Three
-// steps of loads stay in flight behind the MFMAs (with two 64-deep buffers, less than one chunk
-// did, and the kernel waited on its loads).  The four buffers are separate arrays and the loop is
-// unrolled by four, so the compiler can tell the buffers apart and does not wait for outstanding
-// direct loads before the LDS reads of another buffer.
+// ---------------------------------------------------------------- 16-bit, row panels through LDS
+// A workgroup of NW waves owns a 16*MT x 16*NT*NW output tile.  Its waves stand side by side in N:
+// wave w multiplies all 16*MT rows with its own 16*NT columns.  Per 32-deep K step
+//  - the MT row fragments (1 KB half-blocks of the fragment-major layout, contiguous) go into an LDS
+//    ring of four steps by direct global -> LDS loads and are read by every wave;
+//  - each wave loads its own NT weight fragments straight into registers, three steps ahead: no two
+//    waves of the workgroup read the same weights, so LDS would only add a pass.
+// That split is what bounds the kernel: with both operands staged in LDS (256 x 256 or 224 x 256
+// tiles, 8 waves of 112 or 128 x 64) a step read and wrote 88-128 KB of LDS per workgroup for 28-32
+// MFMAs per wave, as long as the MFMAs themselves take; here a 112 x 256 tile moves 7 KB in and 28 KB
+// out.  At 3,584 x 4,096 x 1,024 (random data, weights from HBM): 35.4 us with both operands in LDS,
+// 30.9 us here (973 TFLOP/s); 1,024 x 4,096 x 1,024: 27.7 us (the register kernel that served these
+// rows) -> 13.3.
+//
+// One barrier per step: at step s a wave waits until its own direct loads of step s have landed (those
+// of s + 1 and s + 2 and the weights between them may be in flight), the barrier makes every wave's
+// loads of s visible and says that every wave holds its step s - 1 fragments in registers, so the
+// buffer of s - 1 takes the loads of s + 3.  Two workgroups per CU (or 8 waves) cover each other's
+// barrier and LDS latency.  The four buffers are separate arrays and the loop is unrolled by four, so
+// the compiler can tell them apart and does not wait for outstanding direct loads before LDS reads
+// of another buffer.
 //
 // The MFMAs are inline asm with the accumulators pinned in place in the accumulator registers:
-// compiled from the builtin, the register allocator copied part of the accumulator between
-// register files every chunk, each copy waiting for an MFMA result (measured: a single wave then
-// issues an MFMA every ~32 cycles instead of ~20).  The compiler's hazard checks do not see inside
-// the asm, so the required wait states are explicit at the two points where compiled code touches
-// the accumulators; empty asm statements pin the zeroing before, and the epilogue's reads after,
-// those waits.
+// compiled from the builtin, the register allocator moved accumulators between register files in the
+// loop (and spilled them at 112 rows).  The compiler's hazard checks do not see inside the asm, so the
+// required wait states are explicit at the two points where compiled code touches the accumulators;
+// empty asm statements pin the zeroing before, and the epilogue's reads after, those waits.
 
-// 16 bytes per lane from global memory straight into LDS at dst + 16 * lane (dst wave-uniform).
-// (A plain function: inside a lambda of a kernel template the host pass drops the kernel's stub.)
-__device__ __forceinline__ void lds_direct16(const bf16* src, bf16* dst) {
-    __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+// Buffer resource of `bytes` bytes at p: loads past them return zeros.  (Buffer loads rather than
+// global ones: the compiler counts a global -> LDS load as one that may be flat, after which it waits
+// for every outstanding load, not for the one it needs; and the step's offset is a scalar operand.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+// 16 bytes per lane from byte voff + soff of the buffer straight into LDS at dst + 16 * lane (dst
+// wave-uniform).  (Plain functions: inside a lambda of a kernel template the host pass drops the
+// kernel's stub.)
+__device__ __forceinline__ void lds_buffer16(__amdgpu_buffer_rsrc_t r, int voff, int soff, bf16* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ uint4 ld_buffer16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
 template <int NT, int MT>
@@ -306,22 +324,16 @@ __device__ __forceinline__ float act_fast(float x) {
     else return apply_act(x, ACT);
 }
 
-// Waves form a 2 x 4 grid; each owns 16*MT x 16*NT (AB = 16: 256-row tiles, 128 x 16*NT per wave,
-// NT = 4: 128 pinned accumulator registers; with about 120 vector registers two waves fit per
-// SIMD).  Narrower tiles (NT 3, 2), 224-row tiles (AB = 14, 112 rows per wave) and 128-row tiles
-// (AB = 8, 64 rows per wave) give more workgroups where 256 x 256 tiles would leave CUs idle
-// (3,584 rows = 14 x 256 = 16 x 224: 224-row tiles turn 224 workgroups into 256).  The MFMA operands are swapped (weights as
-// the row operand), so each 16 x 16 accumulator holds C^T: a lane has 4 consecutive output columns
-// of one row, and the epilogue writes 16 bytes (fp32) or 8 bytes (bf16, row-major or
-// fragment-major) per lane.
-template <int NT, int EPI, int ACT, bool H = false, bool BIAS = false, int AB = 16>
-__global__ __launch_bounds__(512, 1) void gemm_bf16_lds_kernel(GemmArgs a) {
-    static_assert(AB == 16 || AB == 14 || AB == 8, "256-, 224- or 128-row tiles");
-    constexpr int MT = AB / 2, BB = 4 * NT;                  // wave row tiles; W blocks (16 columns each) per tile
-    constexpr int TR = 16 * AB;                              // tile rows
-    constexpr int NBLK = AB + BB;                            // 1 KB half-blocks per 32-deep K step
-    constexpr int STAGE = NBLK * 512;                        // halves per LDS stage
-    constexpr int CPS = (NBLK + 7) / 8, CMIN = NBLK / 8;     // direct loads per wave per step (max, min)
+// Row panels that consecutive workgroups of an XCD share before they move to the next columns: an
+// XCD's 32 tiles then cover 4 row panels x 8 column panels, whose operands are a third of those of
+// 1 x 32 (17.7 -> 16.7 us at 1,024 x 4,096 x 1,024, measured with both operands in LDS).
+constexpr int PANEL_GROUP = 4;
+
+template <int MT, int NT, int NW, int EPI, int ACT, bool BIAS>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_panel_kernel(GemmArgs a) {
+    constexpr int TR = 16 * MT, BB = NT * NW;                // tile rows; W blocks (16 columns each) per tile
+    constexpr int STAGE = MT * 512;                          // halves per LDS stage
+    constexpr int CPS = (MT + NW - 1) / NW;                  // direct loads per wave per step
     __shared__ __attribute__((aligned(16))) bf16 st0[STAGE];
     __shared__ __attribute__((aligned(16))) bf16 st1[STAGE];
     __shared__ __attribute__((aligned(16))) bf16 st2[STAGE];
@@ -329,185 +341,147 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_lds_kernel(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) int32_t rtab[EPI == EPI_QKV_RING ? TR : 4];    // QKV: ring row offsets
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool extra = CPS > CMIN && wave + 8 * CMIN < NBLK;   // this wave copies CPS blocks per step, else CMIN
-    const int wm = wave >> 2, wn = wave & 3;
     const int r16 = lane & 15, g = lane >> 4;
-    const int nN = a.N / (64 * NT), nM = (a.M + TR - 1) / TR;
+    const int nN = a.N / (16 * BB), nM = (a.M + TR - 1) / TR;
     const int ks = a.ksplit;
     const int t = xcd_tile(blockIdx.x, nN * nM * ks);
     const int kz = t % ks, tile = t / ks;
-    const int mb = tile / nN, nb = tile % nN;
+    const int grp = tile / (PANEL_GROUP * nN), rem = tile - grp * PANEL_GROUP * nN;
+    const int gm = min(PANEL_GROUP, nM - grp * PANEL_GROUP);
+    const int mb = grp * PANEL_GROUP + rem % gm, nb = rem / gm;
     const int nk = a.K / 64, kper = nk / ks, kc0 = kz * kper;
-    const int nsteps = 2 * kper;                             // 32-deep K steps of this split
+    const int n = 2 * kper;                                  // 32-deep K steps of this split: a multiple of 4
     const int rtiles = (a.M + 15) / 16;
     const bf16* A = static_cast<const bf16*>(a.A);
     const bf16* W = static_cast<const bf16*>(a.W);
+    const int lo = lane * 8;
+    const int ct0 = (nb * NW + wave) * NT;                   // first column tile of this wave
 
-    // Wave w copies the 1 KB half-blocks u = w + 8j of each step: A's row tiles for u < AB, then W's.
-    int soff[CPS];
+    if constexpr (EPI == EPI_QKV_RING) {
+        // the ring offsets of the tile's TR rows (the table is padded past the last row)
+        for (int i = tid; i < TR; i += 64 * NW) rtab[i] = a.ring.rows[mb * TR + i];
+    }
+    // Wave w copies the row fragments w + NW j of each step (past the panel: its last one again) and
+    // loads the column tiles ct0 + j.  Row tiles past the last one are clamped: computed, not stored.
+    const int rt0 = mb * MT, rts = min(MT, rtiles - rt0);
+    const __amdgpu_buffer_rsrc_t ra = buffer_at(A + (((int64_t)rt0 * nk + kc0) << 10), (rts * nk - kc0) * 2048);
+    const __amdgpu_buffer_rsrc_t rw = buffer_at(W + (((int64_t)nb * BB * nk + kc0) << 10), (BB * nk - kc0) * 2048);
+    int aoff[CPS], adst[CPS], woff[NT];
 #pragma unroll
     for (int j = 0; j < CPS; j++) {
-        const int u = wave + 8 * j;
-        int o = 0;
-        if (u < AB) o = (min(mb * AB + u, rtiles - 1) * nk + kc0) << 10;     // clamped rows: not stored
-        else if (u < NBLK) o = ((nb * BB + u - AB) * nk + kc0) << 10;
-        soff[j] = o;
+        const int u = min(wave + NW * j, MT - 1);
+        aoff[j] = min(u, rts - 1) * nk * 2048;
+        adst[j] = u * 512;
     }
-    const int lo = lane * 8;
-    auto copy_step = [&](int s, bf16* dst) __attribute__((always_inline)) {
-        const int kofs = ((s >> 1) << 10) + (s & 1) * 512;
 #pragma unroll
-        for (int j = 0; j < CPS; j++) {
-            const int u = wave + 8 * j;
-            if (j < CMIN || u < NBLK) lds_direct16((u < AB ? A : W) + soff[j] + kofs + lo, dst + u * 512);
-        }
-    };
+    for (int j = 0; j < NT; j++) woff[j] = (wave * NT + j) * nk * 2048;
 
+    uint4 w[4][NT], fa[MT];
+    auto load_step = [&](int s, bf16* dst, uint4 (&wd)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < CPS; j++) lds_buffer16(ra, lane * 16, aoff[j] + s * 1024, dst + adst[j]);
+#pragma unroll
+        for (int j = 0; j < NT; j++) wd[j] = ld_buffer16(rw, lane * 16, woff[j] + s * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+    };
     f32x4_t acc[NT][MT];
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
         for (int i = 0; i < MT; i++) acc[j][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int aoff = (wm * MT) * 512 + lo, boff = (AB + wn * NT) * 512 + lo;
-    // Two fragment register sets: the MFMAs of step s run on one while the LDS reads of step s + 1
-    // fill the other.
-    uint4 fa0[MT], fb0[NT], fa1[MT], fb1[NT];
-    auto read_to = [&](const bf16* buf, uint4 (&xa)[MT], uint4 (&xb)[NT]) __attribute__((always_inline)) {
+    // Step s in buffer cur; the loads of step s + 3 go to nxt / wn (LAST: there are none, and every
+    // outstanding load is waited for).
+    auto step = [&](int s, const bf16* cur, const uint4 (&wc)[NT], bf16* nxt, uint4 (&wn)[NT], auto last)
+        __attribute__((always_inline)) {
+        constexpr bool LAST = decltype(last)::value;
+        // issued after this wave's direct loads of s: the weights of s, then the groups of s + 1, s + 2
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(LAST ? 0 : NT + 2 * (CPS + NT)));
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < MT; i++) xa[i] = *reinterpret_cast<const uint4*>(buf + aoff + i * 512);
-#pragma unroll
-        for (int j = 0; j < NT; j++) xb[j] = *reinterpret_cast<const uint4*>(buf + boff + j * 512);
-    };
-    auto mma = [&](const uint4 (&xa)[MT], const uint4 (&xb)[NT]) __attribute__((always_inline)) {
+        for (int i = 0; i < MT; i++) fa[i] = *reinterpret_cast<const uint4*>(cur + i * 512 + lo);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!LAST) load_step(s + 3, nxt, wn);
+        // (operands swapped, weights as the row operand: each 16 x 16 accumulator holds C^T, so a lane
+        // has 4 consecutive output columns of one row)
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
             for (int i = 0; i < MT; i++)
-                if constexpr (H)
-                    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
-                                 : "+a"(acc[j][i]) : "v"(as_f16x8(xb[j])), "v"(as_f16x8(xa[i])));
-                else
-                    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                                 : "+a"(acc[j][i]) : "v"(as_bf16x8(xb[j])), "v"(as_bf16x8(xa[i])));
-    };
-    // This wave's loads of a step have landed once at most `later` steps' loads (issued after it)
-    // are outstanding: CPS or CMIN direct loads per step for this wave.
-    auto wait_landed = [&](int later) __attribute__((always_inline)) {
-        if (extra) {
-            if (later >= 3) __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * CPS));
-            else if (later == 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * CPS));
-            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(CPS));
-            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        } else {
-            if (later >= 3) __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * CMIN));
-            else if (later == 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * CMIN));
-            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(CMIN));
-            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        }
-    };
-    // QKV split store: the ring offsets of the tile's TR rows (the table is padded past the last row)
-    if constexpr (EPI == EPI_QKV_RING) {
-        if (wave == 0 && lane < TR / 4) lds_direct16_rows(a.ring.rows + mb * TR + 4 * lane, rtab);
-    }
-    // Four-stage ring of 32-deep K steps, fragments one step ahead.  At step s: wait until this
-    // wave's loads of step s + 1 have landed and its LDS reads of step s are done; a barrier makes
-    // every wave's loads of s + 1 visible and frees step s's buffer (every wave holds its step-s
-    // fragments in registers); read the step s + 1 fragments, issue the loads of step s + 4 into
-    // step s's buffer, and multiply step s.  So the LDS reads of one step overlap the MFMAs of the
-    // previous one, and three steps of loads stay in flight behind them.
-    copy_step(0, st0);
-    if (1 < nsteps) copy_step(1, st1);
-    if (2 < nsteps) copy_step(2, st2);
-    if (3 < nsteps) copy_step(3, st3);
-    wait_landed(min(3, nsteps - 1));
-    __builtin_amdgcn_s_barrier();
-    __asm__ volatile("" ::: "memory");
-    read_to(st0, fa0, fb0);
-    pin_acc(acc);
-    asm volatile("s_nop 7");                                 // accumulator zeroing -> first MFMA
-    auto step = [&](int s, const uint4 (&ca)[MT], const uint4 (&cb)[NT], uint4 (&na)[MT], uint4 (&nb)[NT],
-                    const bf16* nbuf, bf16* cbuf) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);                  // lgkmcnt(0): this wave's step-s reads are done
-        if (s + 1 < nsteps) {
-            wait_landed(min(s + 3, nsteps - 1) - (s + 1));
-            __builtin_amdgcn_s_barrier();                    // every wave's loads of step s + 1; step s's buffer free
-            __asm__ volatile("" ::: "memory");
-            read_to(nbuf, na, nb);
-            __builtin_amdgcn_sched_barrier(0);
-            if (s + 4 < nsteps) copy_step(s + 4, cbuf);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        mma(ca, cb);
+                asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
+                             : "+a"(acc[j][i]) : "v"(as_f16x8(wc[j])), "v"(as_f16x8(fa[i])));
         __builtin_amdgcn_sched_barrier(0);
     };
-    for (int s = 0; s < nsteps; s += 4) {
-        step(s, fa0, fb0, fa1, fb1, st1, st0);
-        if (s + 1 < nsteps) step(s + 1, fa1, fb1, fa0, fb0, st2, st1);
-        if (s + 2 < nsteps) step(s + 2, fa0, fb0, fa1, fb1, st3, st2);
-        if (s + 3 < nsteps) step(s + 3, fa1, fb1, fa0, fb0, st0, st3);
+    load_step(0, st0, w[0]);
+    load_step(1, st1, w[1]);
+    load_step(2, st2, w[2]);
+    pin_acc(acc);
+    asm volatile("s_nop 7");                                 // accumulator zeroing -> first MFMA
+    const std::false_type more{};
+    const std::true_type last{};
+    int s = 0;
+    for (; s + 4 < n; s += 4) {
+        step(s, st0, w[0], st3, w[3], more);
+        step(s + 1, st1, w[1], st0, w[0], more);
+        step(s + 2, st2, w[2], st1, w[1], more);
+        step(s + 3, st3, w[3], st2, w[2], more);
     }
+    step(s, st0, w[0], st3, w[3], more);
+    step(s + 1, st1, w[1], st0, w[0], last);
+    step(s + 2, st2, w[2], st1, w[1], last);
+    step(s + 3, st3, w[3], st2, w[2], last);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7");   // last MFMA results -> epilogue reads
     pin_acc(acc);
 
     // acc[j][i] is tile (column tile j, row tile i) transposed: lane holds row 16*rt + r16 and the
     // 4 columns 16*ct + 4*g + e (e < 4).
-    if constexpr (EPI == EPI_GLU) {
-        // column tiles j (values) and j + 1 (gates) of channels 16 ((nb BB + wn NT + j) / 2) ..
-        static_assert(NT % 2 == 0, "value and gate tiles in pairs");
-#pragma unroll
-        for (int i = 0; i < MT; i++) {
-            const int64_t m = (int64_t)(mb * AB + wm * MT + i) * 16 + r16;
-            if (m >= a.M) continue;
-#pragma unroll
-            for (int j = 0; j < NT; j += 2) {
-                const int c = ((nb * BB + wn * NT + j) / 2) * 16 + g * 4;
-                const f32x4_t vv = acc[j][i], vg = acc[j + 1][i];
-                uint2 o;
-                o.x = (uint32_t)to16<H>(vv[0] * sigmoidf(vg[0])) | ((uint32_t)to16<H>(vv[1] * sigmoidf(vg[1])) << 16);
-                o.y = (uint32_t)to16<H>(vv[2] * sigmoidf(vg[2])) | ((uint32_t)to16<H>(vv[3] * sigmoidf(vg[3])) << 16);
-                *reinterpret_cast<uint2*>(static_cast<bf16*>(a.C) + m * a.ldc + c) = o;
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < MT; i++) {
-        const int64_t m = (int64_t)(mb * AB + wm * MT + i) * 16 + r16;
+        const int64_t m = (int64_t)(mb * MT + i) * 16 + r16;
         if (m >= a.M) continue;
+        if constexpr (EPI == EPI_GLU) {
+            // column tiles j (values) and j + 1 (gates) of channels 8 (ct0 + j) ..
+            static_assert(NT % 2 == 0, "value and gate tiles in pairs");
+#pragma unroll
+            for (int j = 0; j < NT; j += 2) {
+                const int c = (ct0 + j) / 2 * 16 + g * 4;
+                const f32x4_t vv = acc[j][i], vg = acc[j + 1][i];
+                *reinterpret_cast<uint2*>(static_cast<bf16*>(a.C) + m * a.ldc + c) =
+                    pack4(vv[0] * sigmoidf(vg[0]), vv[1] * sigmoidf(vg[1]), vv[2] * sigmoidf(vg[2]), vv[3] * sigmoidf(vg[3]));
+            }
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < NT; j++) {
-            const int n = (nb * BB + wn * NT + j) * 16 + g * 4;
+            const int c = (ct0 + j) * 16 + g * 4;
             f32x4_t v = acc[j][i];
-            if constexpr (BIAS) {
-                if (kz == 0) v += *reinterpret_cast<const f32x4_t*>(a.bias + n);
-            }
+            if constexpr (BIAS) v += *reinterpret_cast<const f32x4_t*>(a.bias + c);
             if constexpr (EPI == EPI_PARTIAL) {
-                *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.C) + ((int64_t)kz * a.M + m) * a.ldc + n) =
-                    v * a.out_scale;
-            } else if constexpr (EPI == EPI_STORE_F32) {
-                f32x4_t o;
+                *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.C) + ((int64_t)kz * a.M + m) * a.ldc + c) = v * a.out_scale;
+                continue;
+            }
+            f32x4_t o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = apply_act(v[e], ACT) * a.out_scale;
-                *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.C) + m * a.ldc + n) = o;
+            for (int e = 0; e < 4; e++) o[e] = act_fast<ACT>(v[e]) * a.out_scale;
+            if constexpr (EPI == EPI_STORE_F32) {
+                *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.C) + m * a.ldc + c) = o;
             } else {
-                uint2 o;
-                o.x = (uint32_t)to16<H>(act_fast<ACT>(v[0]) * a.out_scale) | ((uint32_t)to16<H>(act_fast<ACT>(v[1]) * a.out_scale) << 16);
-                o.y = (uint32_t)to16<H>(act_fast<ACT>(v[2]) * a.out_scale) | ((uint32_t)to16<H>(act_fast<ACT>(v[3]) * a.out_scale) << 16);
+                uint2 h = pack4(o[0], o[1], o[2], o[3]);
                 bf16* dst;
                 if constexpr (EPI == EPI_QKV_RING) {   // 4 columns of one head: contiguous in the ring row
-                    dst = n < a.ring.H * 128 ? static_cast<bf16*>(a.C) + m * a.ldc + n
-                                             : qkv_ring_dst(a.ring, rtab[(wm * MT + i) * 16 + r16], n);
+                    dst = c < a.ring.H * 128 ? static_cast<bf16*>(a.C) + m * a.ldc + c
+                                             : qkv_ring_dst(a.ring, rtab[i * 16 + r16], c);
                 } else if constexpr (EPI == EPI_SUBFLAT) {   // 4 columns: contiguous in the fragment block
                     bool masked;
-                    const int64_t d = subflat_dst(a, m, n, masked);
+                    const int64_t d = subflat_dst(a, m, c, masked);
                     if (d < 0) continue;
-                    if (masked) o = make_uint2(0, 0);
+                    if (masked) h = make_uint2(0, 0);
                     dst = static_cast<bf16*>(a.C) + d;
                 } else {
-                    dst = static_cast<bf16*>(a.C) + (EPI == EPI_STORE_FRAG ? frag_index(m, n, a.N / 64) : m * a.ldc + n);
+                    dst = static_cast<bf16*>(a.C) + (EPI == EPI_STORE_FRAG ? frag_index(m, c, a.N / 64) : m * a.ldc + c);
                 }
-                *reinterpret_cast<uint2*>(dst) = o;
+                *reinterpret_cast<uint2*>(dst) = h;
             }
         }
     }
@@ -680,51 +654,25 @@ int launch_gemm_f32_small(const GemmArgs& a, int ks, hipStream_t st) {
 
 // ---------------------------------------------------------------- launch
 
-template <int MT, int WK, int NT, int EPI, int ACT, bool H = false, bool BIAS = false>
-static int launch_bf16_cfg(GemmArgs a, int ksplit, hipStream_t st) {
+template <int MT, int WK, int NT, int EPI, int ACT, bool BIAS = false>
+static int launch_reg(GemmArgs a, int ksplit, hipStream_t st) {
     if (a.N % (16 * NT) != 0 || ksplit < 1 || a.K % (64 * ksplit) != 0 || a.K / (64 * ksplit) < WK) return -2;
     if (ksplit > 1 && EPI != EPI_PARTIAL) return -2;
     if (EPI == EPI_STORE_FRAG && a.N % 64 != 0) return -2;
     a.ksplit = ksplit;
     const int tiles = (a.N / (16 * NT)) * ((a.M + 16 * MT - 1) / (16 * MT)) * ksplit;
-    hipLaunchKernelGGL((gemm_bf16_kernel<MT, WK, EPI, ACT, NT, H, BIAS>), dim3(tiles), dim3(64 * WK), 0, st, a);
+    hipLaunchKernelGGL((gemm_bf16_kernel<MT, WK, EPI, ACT, NT, BIAS>), dim3(tiles), dim3(64 * WK), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <int NT, int EPI, int ACT, bool H = false, bool BIAS = false, int AB = 16>
-static int launch_lds_cfg(GemmArgs a, int ksplit, hipStream_t st) {
-    if (a.N % (64 * NT) != 0 || ksplit < 1 || a.K % (64 * ksplit) != 0 || a.ldc % 4 != 0) return -2;
+template <int MT, int NT, int NW, int EPI, int ACT, bool BIAS>
+static int launch_panel(GemmArgs a, int ksplit, hipStream_t st) {
+    if (a.N % (16 * NT * NW) != 0 || ksplit < 1 || a.K % (128 * ksplit) != 0 || a.ldc % 4 != 0) return -2;
     if (ksplit > 1 && EPI != EPI_PARTIAL) return -2;
-    if ((int64_t)((a.M + 15) / 16) * a.K * 16 >= (1ll << 31) || (int64_t)a.N * a.K >= (1ll << 31)) return -2;
     a.ksplit = ksplit;
-    const int tiles = (a.N / (64 * NT)) * ((a.M + 16 * AB - 1) / (16 * AB)) * ksplit;
-    hipLaunchKernelGGL((gemm_bf16_lds_kernel<NT, EPI, ACT, H, BIAS, AB>), dim3(tiles), dim3(512), 0, st, a);
+    const int tiles = (a.N / (16 * NT * NW)) * ((a.M + 16 * MT - 1) / (16 * MT)) * ksplit;
+    hipLaunchKernelGGL((gemm_panel_kernel<MT, NT, NW, EPI, ACT, BIAS>), dim3(tiles), dim3(64 * NW), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-template <int NT, int EPI, bool H, int AB>
-static int launch_lds_epi(const GemmArgs& a, int ks, hipStream_t st) {
-    switch (a.act) {
-        case ACT_NONE: return launch_lds_cfg<NT, EPI, ACT_NONE, H, false, AB>(a, ks, st);
-        case ACT_SILU: return launch_lds_cfg<NT, EPI, ACT_SILU, H, false, AB>(a, ks, st);
-        case ACT_RELU: return launch_lds_cfg<NT, EPI, ACT_RELU, H, false, AB>(a, ks, st);
-        default: return -2;
-    }
-}
-
-template <int NT, bool H, int AB>
-static int launch_lds_act(const GemmArgs& a, int ks, hipStream_t st) {
-    switch (a.epi) {
-        case EPI_PARTIAL: return a.act == ACT_NONE ? launch_lds_cfg<NT, EPI_PARTIAL, ACT_NONE, H, false, AB>(a, ks, st) : -2;
-        case EPI_STORE_F32: return launch_lds_epi<NT, EPI_STORE_F32, H, AB>(a, ks, st);
-        case EPI_STORE_FRAG: return launch_lds_epi<NT, EPI_STORE_FRAG, H, AB>(a, ks, st);
-        case EPI_STORE: return launch_lds_epi<NT, EPI_STORE, H, AB>(a, ks, st);
-        case EPI_QKV_RING: return launch_lds_cfg<NT, EPI_QKV_RING, ACT_NONE, H, false, AB>(a, ks, st);
-        case EPI_GLU:
-            if constexpr (NT % 2 == 0) return a.act == ACT_NONE ? launch_lds_cfg<NT, EPI_GLU, ACT_NONE, H, false, AB>(a, ks, st) : -2;
-            return -2;
-        default: return -2;
-    }
 }
 
 static int device_cus() {
@@ -739,230 +687,154 @@ static int device_cus() {
     return cus;
 }
 
-// Tile shape (256 or 128 rows, NT: 64*NT columns) and K splits of the LDS-staged kernel for one
-// projection.  Cost model: rounds of workgroups over the CUs (the wave quantisation: a second,
-// partly filled round costs a whole round) x the per-workgroup MFMA work, scaled by the per-flop
-// cost of each tile shape (256 rows: NT 4 1.00, 3 1.28, 2 1.36, measured at 3584 rows; 128 rows:
-// 2.0), plus for K splits the fp32 partial slabs they write and the LayerNorm after them reads
-// back (900 units per slab per 3584 x 1024 outputs: a slab's stores come at the end of the one
-// round of workgroups, where nothing hides them, about 2-3 us, and its read in the LayerNorm
-// about 2.5 us).
-// A 128-row tile re-reads each weight panel twice as often as a 256-row one.  Measured on the
-// 24-layer 256-stream x 14-frame step (eager launches, all choices in one process):
-// 8.409 ms with 256-row tiles everywhere; 8.218 ms with linear_out and pointwise_conv2 on 128 x 128
-// tiles (224 workgroups instead of 112 on 256 CUs: 19.7 -> 14.5 us each); 8.209 ms with the
-// subsampling's out projection too; worse with 128-row tiles for q/k/v (+0.134 ms),
-// pointwise_conv1 (+0.126 ms) or ff linear2 (+0.05 ms with 2 splits, more without), which already
-// launch 224 256-row workgroups.  The 128-row cost of 2.0 makes 128-row tiles win only where
-// 256-row tiles leave about half the CUs idle, which is what those runs show.
-// 224-row tiles: each weight panel is re-read 8/7 as often per flop as with 256-row tiles.  At
-// 3,584 rows they give 256 workgroups instead of 224 (ff linear1, q/k/v, pointwise_conv1, ff
-// linear2 with 2 splits); with the fragments read one step ahead that step went 8.02 -> 7.95 ms
-// (the same fragment schedule with 256-row tiles only: 8.05 ms).
-constexpr double C224 = 1.05;
-BigTile big_tile(int M, int N, int K, bool partial, int heights_mask) {
-    static const double cost_256[5] = {0.0, 0.0, 1.36, 1.28, 1.0};
-    static const double cost_128[5] = {0.0, 0.0, 2.0, 2.0, 2.0};
-    const int cus = device_cus();
-    BigTile best{0, 1, 16};
-    double best_cost = 1e300;
-    static const int heights[3] = {16, 14, 8};
-    for (int hi = 0; hi < 3; hi++)
-        for (int nt = 4; nt >= 2; nt--) {
-            if (!(heights_mask & (1 << hi))) continue;
-            const int ab = heights[hi];
-            // per-flop cost: 256-row measured; 224 rows re-read each weight panel 8/7 as often
-            const double pc = ab == 16 ? cost_256[nt] : ab == 14 ? cost_256[nt] * C224 : cost_128[nt];
-            if (N % (64 * nt) != 0) continue;
-            for (int ks = 1; ks <= (partial ? 4 : 1); ks *= 2) {
-                if (K % (64 * ks) != 0 || (ks > 1 && K / ks < 256)) continue;
-                const long tiles = (long)(N / (64 * nt)) * ((M + 16 * ab - 1) / (16 * ab)) * ks;
-                const long rounds = (tiles + cus - 1) / cus;
-                double cost = (double)rounds * (ab / 16.0) * nt * (K / ks) * pc;
-                if (ks > 1) cost += 900.0 * ks * ((double)M * N / (3584.0 * 1024.0));
-                if (cost < best_cost) { best_cost = cost; best = BigTile{nt, ks, ab}; }
-            }
+// The kernel, tile and K splits of one 16-bit GEMM.
+enum Gemm16 : int {
+    REG_64x64,          // gemm_bf16_kernel<4, 4, .., 4>: 4 waves split K
+    REG_64x32,          // gemm_bf16_kernel<4, 4, .., 2>: 4 waves split K
+    PANEL_64x128,       // gemm_panel_kernel<4, 2, 4>
+    PANEL_128x128,      // gemm_panel_kernel<8, 2, 4>
+    PANEL_112x256,      // gemm_panel_kernel<7, 4, 4>
+    REG_128x16,         // gemm_bf16_kernel<8, 2, .., 1>: any N % 16 == 0, K % 128 == 0
+    REG_FEW,            // at most 128 rows: the shapes of launch_few
+};
+struct Plan16 { Gemm16 kind; int ks; };
+
+// Few rows: the waves of a workgroup split K.  Many rows: the tile that fills the CUs.  Between them
+// no tile is best for long (a workgroup more on some CU costs a whole round of K steps), so the
+// choice is a model of each kernel's time,
+//   t = t0 + steps (p + q load) + r load  [us],  load = most workgroups on a CU, steps = 32-deep K steps,
+// fitted to its times at the encoder's seven shapes (N 256-4,096, K 256-4,352) over 130-57,344 rows
+// with weights from HBM; the model's choice is on average 1.5 % slower than the best of the five.
+// The K slabs of a residual projection cost the LayerNorm that adds them, and the stores, about
+// 1.2 us per slab per 1,000 x 1,024 outputs.
+// Measured against what these rows had (128 x 16 register tiles below 2,048 rows, 128/224/256-row
+// tiles with both operands in LDS above), us per launch, random data:
+//   rows                        256          640          1,024        2,048        3,584
+//   ff linear1 (4,096 x 1,024)  11.2 -> 7.9  19.5 -> 12.7 27.7 -> 13.3 21.6 -> 21.0 35.4 -> 30.9
+//   ff linear2 (1,024 x 4,096)  10.8 -> 7.5  25.1 -> 14.7 50.8 -> 15.5 26.1 -> 23.5 36.5 -> 33.8
+//   q/k/v (3,072 x 1,024)        9.3 -> 7.0  14.5 ->  9.3 22.9 -> 12.4 21.0 -> 18.8 30.5 -> 28.2
+//   linear_out (1,024 x 1,024)   4.9 -> 4.0   8.1 ->  6.0 11.0 ->  6.5 12.0 ->  8.7 15.1 -> 13.6
+static Plan16 plan16(int M, int N, int K, int epi) {
+    const bool partial = epi == EPI_PARTIAL;
+    if (M <= 128) return Plan16{REG_FEW, !partial ? 1 : K == 1024 && N % 32 == 0 ? 2 : K % (128 * KSPLIT) == 0 ? KSPLIT : 1};
+    struct Model { Gemm16 kind; int rows, cols, waves_k; double t0, p, q, r; };
+    static const Model models[] = {
+        {REG_64x64, 64, 64, 4, 0.0, 0.0137, 0.0915, 3.151},
+        {REG_64x32, 64, 32, 4, 0.98, 0.0160, 0.0690, 0.752},
+        {PANEL_64x128, 64, 128, 0, 1.05, 0.0926, 0.0925, 1.867},
+        {PANEL_128x128, 128, 128, 0, 0.90, 0.1222, 0.1117, 3.915},
+        {PANEL_112x256, 112, 256, 0, 0.28, 0.1726, 0.1656, 6.654},
+    };
+    const long cus = device_cus();
+    Plan16 best{REG_128x16, partial && K % (128 * KSPLIT) == 0 ? KSPLIT : 1};
+    double best_t = 1e300;
+    for (const Model& m : models)
+        for (int ks = 1; ks <= (partial ? KSPLIT : 1); ks *= 2) {
+            // the panel kernel runs whole groups of four K steps; a register wave needs a 64-deep chunk
+            if (N % m.cols != 0 || K % (128 * ks) != 0 || (ks > 1 && K / ks < 256) || K / (64 * ks) < m.waves_k) continue;
+            const long load = ((long)(N / m.cols) * ((M + m.rows - 1) / m.rows) * ks + cus - 1) / cus;
+            double t = m.t0 + K / (32.0 * ks) * (m.p + m.q * load) + m.r * load;
+            if (partial) t += 1.2 * ks * ((double)M * N / 1024e3);
+            if (t < best_t) { best_t = t; best = Plan16{m.kind, ks}; }
         }
     return best;
 }
 
-int gemm_partial_splits(int M, int N, int K, bool bf16_data) {
-    if (!bf16_data) return 1;
-    if (M >= LDS_MIN_ROWS) {
-        const BigTile bt = big_tile(M, N, K, true, TILE_ALL);
-        if (bt.nt != 0) return bt.ks;
-    }
-    if (M <= 128 && K == 1024 && N % 32 == 0) return 2;   // linear_out, pointwise_conv2 (launch_bf16)
-    return K % (128 * KSPLIT) == 0 ? KSPLIT : 1;
-}
-
-template <int MT, int WK, int NT, int EPI, bool H>
-static int launch_act(const GemmArgs& a, int ks, hipStream_t st) {
-    if (a.act == ACT_SILU) return launch_bf16_cfg<MT, WK, NT, EPI, ACT_SILU, H>(a, ks, st);
-    if (a.act == ACT_NONE) return launch_bf16_cfg<MT, WK, NT, EPI, ACT_NONE, H>(a, ks, st);
-    if (a.act == ACT_RELU) return launch_bf16_cfg<MT, WK, NT, EPI, ACT_RELU, H>(a, ks, st);
-    return -2;
-}
+int gemm_partial_splits(int M, int N, int K) { return plan16(M, N, K, EPI_PARTIAL).ks; }
 
 // Tile shapes measured on MI355X for the streaming step's M <= 128 projections (weights from HBM,
 // 48 rotating copies; the waves of a workgroup split K and share the reduction and the epilogue):
 //   ff linear1 (N 4096, K 1024, fragment out):  MT 2 x NT 4, 8 waves            6.97 -> 5.94 us
-//   q/k/v (N 3072, K 1024, bf16 out):           MT 4 x NT 2, 8 waves            5.77 -> 5.53 us
-//   pointwise_conv1 (N 2048, K 1024, fp32 out): MT 2 x NT 2, 8 waves            4.31 -> 3.76 us
+//   q/k/v (N 3072, K 1024, half out):           MT 4 x NT 2, 8 waves            5.77 -> 5.53 us
+//   pointwise_conv1 (N 2048, K 1024, GLU out):  MT 2 x NT 2, 8 waves            4.31 -> 3.76 us
 //   ff linear2 (N 1024, K 4096, split-K 4):     MT 4 x NT 2, 8 waves            5.91 -> 5.76 us
 //   linear_out, pw2 (N 1024, K 1024):           MT 2 x NT 2, 8 waves, split-K 2 3.40 -> 3.12 us
 //                                               (half the slabs for the LayerNorm that adds them)
+//   subsampling out (N 1024, K 4352, bias):     MT 2 x NT 1, 8 waves: 256 workgroups of 8 or 9 chunks
+//                                               a wave (64 workgroups of 4 waves: ~4 us longer)
 // Wider tiles cut the re-reads of the activation panel; more waves per workgroup put more of a
 // tile's K range in flight at once.
-// Larger M keeps 128-row tiles (MT 8, 2 waves).
-// IEEE-half operands with a bias (the subsampling front-end's GEMMs): fp32 outputs (EPI_STORE_F32),
-// half outputs (EPI_STORE, row-major) or conv.6's flattened rows (EPI_SUBFLAT); no activation or
-// ReLU.  The bias is a template parameter: a runtime-optional bias in the encoder's own GEMMs made
-// their epilogues larger and cost ~2 us per launch at 128 rows.
-template <int EPI, int ACT>
-static int launch_f16(const GemmArgs& a, hipStream_t st) {
-    // (the subsampling's out Linear at 128 rows: K = 4,352 is 68 chunks, 8 or 9 per wave over 256
-    // workgroups of 8 waves; with 4 waves of 17 chunks over 64 workgroups it took ~4 us longer)
-    if (a.M <= 128 && a.N % 16 == 0 && a.K % 64 == 0 && a.K >= 512)
-        return launch_bf16_cfg<2, 8, 1, EPI, ACT, true, true>(a, 1, st);
-    if (a.M <= 128 && a.N % 32 == 0 && a.K % 256 == 0) return launch_bf16_cfg<4, 4, 2, EPI, ACT, true, true>(a, 1, st);
-    // The LDS kernel's 256-row tiles leave most CUs idle below ~64 tiles (the second pointwise conv
-    // of 64 streams x 160 ms: 4,352 x 256 x 256, 34 tiles, 10.5 us; the register kernel's 64 x 32
-    // tiles 6.6 us, 11.7 us once its epilogue wrote the out Linear's flattened rows, 8.2 us with 4
-    // waves of one 64-deep chunk each instead of 2 of two).
-    const BigTile b256 = a.M >= LDS_MIN_ROWS ? big_tile(a.M, a.N, a.K, false, TILE_256) : BigTile{0, 1, 16};
-    if (b256.nt != 0 && (int64_t)((a.M + 255) / 256) * (a.N / (64 * b256.nt)) < 64 && a.N % 32 == 0 && a.K % 128 == 0)
-        return a.K >= 256 ? launch_bf16_cfg<4, 4, 2, EPI, ACT, true, true>(a, 1, st)
-                          : launch_bf16_cfg<4, 2, 2, EPI, ACT, true, true>(a, 1, st);
-    const BigTile bt = a.M >= LDS_MIN_ROWS ? big_tile(a.M, a.N, a.K, false, TILE_256 | TILE_128) : BigTile{0, 1, 16};
-    const int nt = bt.nt;
-    if (a.M >= LDS_MIN_ROWS) {
-        if (bt.ab == 8) {
-            switch (nt) {
-                case 4: return launch_lds_cfg<4, EPI, ACT, true, true, 8>(a, 1, st);
-                case 3: return launch_lds_cfg<3, EPI, ACT, true, true, 8>(a, 1, st);
-                case 2: return launch_lds_cfg<2, EPI, ACT, true, true, 8>(a, 1, st);
-                default: break;
-            }
-        }
-        switch (nt) {
-            case 4: return launch_lds_cfg<4, EPI, ACT, true, true>(a, 1, st);
-            case 3: return launch_lds_cfg<3, EPI, ACT, true, true>(a, 1, st);
-            case 2: return launch_lds_cfg<2, EPI, ACT, true, true>(a, 1, st);
-            default: break;
-        }
+template <int EPI, int ACT, bool BIAS>
+static int launch_few(const GemmArgs& a, int ks, hipStream_t st) {
+    const bool k512 = a.K % (512 * ks) == 0;
+    if constexpr (BIAS) {
+        if (a.K >= 512) return launch_reg<2, 8, 1, EPI, ACT, true>(a, 1, st);
+        if (a.N % 32 == 0 && a.K % 256 == 0) return launch_reg<4, 4, 2, EPI, ACT, true>(a, 1, st);
+    } else if constexpr (EPI == EPI_STORE_FRAG) {
+        if (k512) return launch_reg<2, 8, 4, EPI, ACT>(a, 1, st);
+        return launch_reg<2, 2, 4, EPI, ACT>(a, 1, st);
+    } else if constexpr (EPI == EPI_STORE || EPI == EPI_QKV_RING) {
+        if (a.N % 32 == 0 && k512) return launch_reg<4, 8, 2, EPI, ACT>(a, 1, st);
+    } else if constexpr (EPI == EPI_STORE_F32 || EPI == EPI_GLU) {
+        if (a.N % 32 == 0 && k512) return launch_reg<2, 8, 2, EPI, ACT>(a, 1, st);
+    } else if constexpr (EPI == EPI_PARTIAL) {
+        if (a.N % 32 == 0 && k512)
+            return a.K >= 4096 ? launch_reg<4, 8, 2, EPI, ACT>(a, ks, st) : launch_reg<2, 8, 2, EPI, ACT>(a, ks, st);
+        if (a.K % (128 * ks) == 0) return launch_reg<4, 2, 1, EPI, ACT>(a, ks, st);
     }
-    return launch_bf16_cfg<8, 2, 1, EPI, ACT, true, true>(a, 1, st);
+    return launch_reg<8, 2, EPI == EPI_GLU ? 2 : 1, EPI, ACT, BIAS>(a, ks, st);
 }
 
-template <int EPI>
-static int launch_f16_act(const GemmArgs& a, hipStream_t st) {
-    if (a.act == ACT_NONE) return launch_f16<EPI, ACT_NONE>(a, st);
-    if (a.act == ACT_RELU) return launch_f16<EPI, ACT_RELU>(a, st);
-    return -2;
-}
-
-// The encoder's 16-bit projections: operands (and 16-bit outputs) IEEE half when H, bf16 otherwise;
-// no bias.
-template <bool H>
+template <int EPI, int ACT, bool BIAS>
 static int launch_16(const GemmArgs& a, int ks, hipStream_t st) {
-    if (a.bias != nullptr) return -2;   // the encoder's projections have no bias
-    if (a.M <= 128) {
-        switch (a.epi) {
-            case EPI_STORE_FRAG:
-                if (a.N % 64 == 0 && a.K % 512 == 0) return launch_act<2, 8, 4, EPI_STORE_FRAG, H>(a, ks, st);
-                if (a.N % 64 == 0) return launch_act<2, 2, 4, EPI_STORE_FRAG, H>(a, ks, st);
-                break;
-            case EPI_STORE:
-                if (a.N % 32 == 0 && a.K % 512 == 0) return launch_act<4, 8, 2, EPI_STORE, H>(a, ks, st);
-                break;
-            case EPI_QKV_RING:
-                if (a.N % 32 == 0 && a.K % 512 == 0) return launch_bf16_cfg<4, 8, 2, EPI_QKV_RING, ACT_NONE, H>(a, ks, st);
-                break;
-            case EPI_STORE_F32:
-                if (a.N % 32 == 0 && a.K % 512 == 0) return launch_act<2, 8, 2, EPI_STORE_F32, H>(a, ks, st);
-                break;
-            case EPI_GLU:
-                if (a.K % 512 == 0) return launch_bf16_cfg<2, 8, 2, EPI_GLU, ACT_NONE, H>(a, ks, st);
-                break;
-            case EPI_PARTIAL:
-                if (a.act != ACT_NONE) return -2;
-                if (a.N % 32 == 0 && a.K % (512 * ks) == 0)
-                    return a.K >= 4096 ? launch_bf16_cfg<4, 8, 2, EPI_PARTIAL, ACT_NONE, H>(a, ks, st)
-                                       : launch_bf16_cfg<2, 8, 2, EPI_PARTIAL, ACT_NONE, H>(a, ks, st);
-                if (a.K % (128 * ks) == 0) return launch_bf16_cfg<4, 2, 1, EPI_PARTIAL, ACT_NONE, H>(a, ks, st);
-                break;
-            default: return -2;   // the residual accumulate is an fp32-path epilogue
-        }
+    const Plan16 p = plan16(a.M, a.N, a.K, EPI);
+    if (p.ks != ks) return -2;              // EPI_PARTIAL: the caller sized its slabs by another plan
+    switch (p.kind) {
+        case REG_64x64: return launch_reg<4, 4, 4, EPI, ACT, BIAS>(a, ks, st);
+        case REG_64x32: return launch_reg<4, 4, 2, EPI, ACT, BIAS>(a, ks, st);
+        case PANEL_64x128: return launch_panel<4, 2, 4, EPI, ACT, BIAS>(a, ks, st);
+        case PANEL_128x128: return launch_panel<8, 2, 4, EPI, ACT, BIAS>(a, ks, st);
+        case PANEL_112x256: return launch_panel<7, 4, 4, EPI, ACT, BIAS>(a, ks, st);
+        case REG_FEW: return launch_few<EPI, ACT, BIAS>(a, ks, st);
+        default: return launch_reg<8, 2, EPI == EPI_GLU ? 2 : 1, EPI, ACT, BIAS>(a, ks, st);
     }
-    if (a.M >= LDS_MIN_ROWS) {
-        const BigTile bt = big_tile(a.M, a.N, a.K, a.epi == EPI_PARTIAL, TILE_ALL);
-        if (bt.nt != 0 && (a.epi != EPI_PARTIAL || bt.ks == ks) && (a.epi != EPI_GLU || bt.nt % 2 == 0)) {
-            if (H && bt.ab == 8) {          // 128- and 224-row tiles: instantiated for the encoder's half operands
-                switch (bt.nt) {
-                    case 4: return launch_lds_act<4, true, 8>(a, ks, st);
-                    case 3: return launch_lds_act<3, true, 8>(a, ks, st);
-                    default: return launch_lds_act<2, true, 8>(a, ks, st);
-                }
-            }
-            if (H && bt.ab == 14) {
-                switch (bt.nt) {
-                    case 4: return launch_lds_act<4, true, 14>(a, ks, st);
-                    case 3: return launch_lds_act<3, true, 14>(a, ks, st);
-                    default: return launch_lds_act<2, true, 14>(a, ks, st);
-                }
-            }
-            switch (bt.nt) {
-                case 4: return launch_lds_act<4, H, 16>(a, ks, st);
-                case 3: return launch_lds_act<3, H, 16>(a, ks, st);
-                default: return launch_lds_act<2, H, 16>(a, ks, st);
-            }
-        }
-    }
-    switch (a.epi) {
-        case EPI_PARTIAL: return a.act == ACT_NONE ? launch_bf16_cfg<8, 2, 1, EPI_PARTIAL, ACT_NONE, H>(a, ks, st) : -2;
-        case EPI_STORE_F32: return launch_act<8, 2, 1, EPI_STORE_F32, H>(a, ks, st);
-        case EPI_STORE_FRAG: return launch_act<8, 2, 1, EPI_STORE_FRAG, H>(a, ks, st);
-        case EPI_STORE: return launch_act<8, 2, 1, EPI_STORE, H>(a, ks, st);
-        case EPI_QKV_RING: return launch_bf16_cfg<8, 2, 1, EPI_QKV_RING, ACT_NONE, H>(a, ks, st);
-        case EPI_GLU: return a.act == ACT_NONE ? launch_bf16_cfg<8, 2, 2, EPI_GLU, ACT_NONE, H>(a, ks, st) : -2;
+}
+
+template <int EPI, bool BIAS>
+static int launch_act(const GemmArgs& a, hipStream_t st) {
+    switch (a.act) {
+        case ACT_NONE: return launch_16<EPI, ACT_NONE, BIAS>(a, 1, st);
+        case ACT_SILU: return BIAS ? -2 : launch_16<EPI, ACT_SILU, false>(a, 1, st);
+        case ACT_RELU: return launch_16<EPI, ACT_RELU, BIAS>(a, 1, st);
         default: return -2;
     }
 }
 
-static int launch_bf16(const GemmArgs& a, int ks, hipStream_t st) {
-    if (a.f16 && a.bias != nullptr) {
-        // the subsampling front-end's GEMMs: IEEE half with a bias
-        if (ks != 1) return -2;
-        switch (a.epi) {
-            case EPI_STORE_F32: return launch_f16_act<EPI_STORE_F32>(a, st);
-            case EPI_STORE: return launch_f16_act<EPI_STORE>(a, st);
-            case EPI_SUBFLAT:
-                if (!a.flat.vlen || a.flat.T3 < 1 || a.flat.F3 < 1 || a.flat.drop < 0 || a.flat.T != a.flat.T3 - a.flat.drop ||
-                    (int64_t)a.M >= (1ll << 31) ||
-                    (int64_t)a.M != (int64_t)a.M / (a.flat.T3 * a.flat.F3) * a.flat.T3 * a.flat.F3 || (a.flat.F3 * a.N) % 64)
-                    return -2;
-                return launch_f16_act<EPI_SUBFLAT>(a, st);
-            default: return -2;
-        }
+// The encoder's projections have no bias; the subsampling front-end's GEMMs have one (a template
+// parameter: a runtime-optional bias in the encoder's own GEMMs made their epilogues larger and cost
+// ~2 us per launch at 128 rows).
+static int launch_half(const GemmArgs& a, hipStream_t st) {
+    const bool bias = a.bias != nullptr;
+    switch (a.epi) {
+        case EPI_STORE: return bias ? launch_act<EPI_STORE, true>(a, st) : launch_act<EPI_STORE, false>(a, st);
+        case EPI_STORE_F32: return bias ? launch_act<EPI_STORE_F32, true>(a, st) : launch_act<EPI_STORE_F32, false>(a, st);
+        case EPI_SUBFLAT: return bias ? launch_act<EPI_SUBFLAT, true>(a, st) : -2;
+        default: break;
     }
-    return a.f16 ? launch_16<true>(a, ks, st) : launch_16<false>(a, ks, st);
+    if (bias) return -2;
+    switch (a.epi) {
+        case EPI_STORE_FRAG: return a.N % 64 == 0 ? launch_act<EPI_STORE_FRAG, false>(a, st) : -2;
+        case EPI_QKV_RING: return launch_16<EPI_QKV_RING, ACT_NONE, false>(a, 1, st);
+        case EPI_GLU: return launch_16<EPI_GLU, ACT_NONE, false>(a, 1, st);
+        case EPI_PARTIAL: return a.act == ACT_NONE ? launch_16<EPI_PARTIAL, ACT_NONE, false>(a, a.ksplit, st) : -2;
+        default: return -2;   // the residual accumulate is an fp32-path epilogue
+    }
 }
 
-int launch_gemm(const GemmArgs& a, bool bf16_data, hipStream_t st) {
+int launch_gemm(const GemmArgs& a, bool half_data, hipStream_t st) {
     if (a.M <= 0 || a.N <= 0 || a.K <= 0) return -2;
     // GLU pairs: 16-bit only, no activation, whole 32-column value/gate blocks, half the columns out
-    if (a.epi == EPI_GLU && (!bf16_data || a.act != ACT_NONE || a.bias || a.N % 32 != 0 || a.ldc < a.N / 2 || a.ldc % 4))
+    if (a.epi == EPI_GLU && (!half_data || a.act != ACT_NONE || a.bias || a.N % 32 != 0 || a.ldc < a.N / 2 || a.ldc % 4))
         return -2;
     if (a.epi == EPI_QKV_RING) {
         // 16-bit only, no activation; the rows are whole streams of T frames; every ring row written
         // is outside the step's window (L + T <= R)
         const QkvRing& r = a.ring;
-        if (!bf16_data || a.act != ACT_NONE || a.bias || !r.kring || !r.vring || !r.rows || r.T < 1 || r.H < 1 ||
+        if (!half_data || a.act != ACT_NONE || a.bias || !r.kring || !r.vring || !r.rows || r.T < 1 || r.H < 1 ||
             a.N != 3 * r.H * 128 || a.M % r.T != 0 || r.L + r.T > r.R || a.ldc < r.H * 128)
             return -2;
     }
-    if (!bf16_data) {
+    if (!half_data) {
         if (a.epi == EPI_STORE_FRAG) return -2;
         const int ks = a.epi == EPI_PARTIAL ? a.ksplit : 1;
         if (ks < 1 || ks > 64) return -2;
@@ -971,7 +843,13 @@ int launch_gemm(const GemmArgs& a, bool bf16_data, hipStream_t st) {
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     if (a.K % 128 != 0) return -2;
-    return launch_bf16(a, a.epi == EPI_PARTIAL ? a.ksplit : 1, st);
+    if (a.epi == EPI_SUBFLAT) {
+        const SubFlat& f = a.flat;
+        if (!f.vlen || f.T3 < 1 || f.F3 < 1 || f.drop < 0 || f.T != f.T3 - f.drop || a.M % (f.T3 * f.F3) != 0 ||
+            (f.F3 * a.N) % 64)
+            return -2;
+    }
+    return launch_half(a, st);
 }
 
 }  // namespace ud

@@ -119,7 +119,7 @@ struct QkvRing {
     const int32_t* rows;            // [M + 256]: ring element offset per output row (padded)
     int T, L, R, H;
 };
-// bf16: A [M, K] and W [N, K] in fragment-major layout (lda/ldw unused); M may be any size, the
+// half_data: A [M, K] and W [N, K] IEEE half in fragment-major layout (lda/ldw unused); M may be any size, the
 // A buffer holding ceil(M/16)*16 rows.  fp32: row-major with leading dimensions lda/ldw/ldc.
 struct GemmArgs {
     const void* A; const void* W; void* C;
@@ -127,30 +127,20 @@ struct GemmArgs {
     int epi, act;
     float out_scale;
     int ksplit;                     // EPI_PARTIAL: K splits chosen by the caller (gemm_partial_splits)
-    const float* bias;              // [N] added before the activation: fp32 path (optional) and the
-                                    // IEEE-half path (required); not the bf16 path
-    int f16;                        // 16-bit path: operands (and 16-bit outputs) are IEEE half
-                                    // instead of bf16
+    const float* bias;              // [N] added before the activation (optional)
     QkvRing ring;                   // EPI_QKV_RING only
     SubFlat flat;                   // EPI_SUBFLAT only
 };
-int launch_gemm(const GemmArgs& a, bool bf16_data, hipStream_t st);
+int launch_gemm(const GemmArgs& a, bool half_data, hipStream_t st);
 // fp32 GEMM for few rows (tens) on the fp32 MFMA: EPI_PARTIAL with ks K splits (slabs
 // [ks][M][ldc]) or EPI_STORE (ks = 1, optional bias, act).  K % (16 ks) == 0, lda and ldw multiples
 // of 4, A and W 16-byte aligned; any M and N.
 int launch_gemm_f32_small(const GemmArgs& a, int ks, hipStream_t st);
-// Most K splits of a bf16 residual projection (partial slabs the workspace holds).
+// Most K splits of a 16-bit residual projection (partial slabs the workspace holds).
 constexpr int KSPLIT = 4;
-// Rows from which the bf16 projections use the LDS-staged kernel (256- or 128-row tiles).
-constexpr int LDS_MIN_ROWS = 2048;
-struct BigTile { int nt, ks, ab; };   // 16*ab-row x 64*nt-column tiles (ab 16, 14 or 8), ks K splits
-                                      // (nt 0: shape not supported)
-// heights_mask: the tile heights that are candidates (TILE_256 | TILE_224 | TILE_128)
-constexpr int TILE_256 = 1, TILE_224 = 2, TILE_128 = 4, TILE_ALL = 7;
-BigTile big_tile(int M, int N, int K, bool partial, int heights_mask);
-// K splits (partial slabs) a residual projection of this shape writes; launch_gemm expects it in
-// GemmArgs::ksplit for EPI_PARTIAL.
-int gemm_partial_splits(int M, int N, int K, bool bf16_data);
+// K splits (partial slabs) a 16-bit residual projection of this shape writes; launch_gemm expects it
+// in GemmArgs::ksplit for EPI_PARTIAL.
+int gemm_partial_splits(int M, int N, int K);
 
 // ---------------------------------------------------------------- LayerNorm / conv / misc
 // Pending residual update: nparts fp32 slabs [rows, D] (stride rows*D) that a split-K residual
