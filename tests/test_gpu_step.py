@@ -417,3 +417,15 @@ def test_step_bf16_projection_tiles(gpu, orc, S, T):
     for got, ref in res:
         harness.assert_bf16_close(got, ref, "%d x %d" % (S, T))
     enc.close()
+
+
+@pytest.mark.parametrize("S,T,ff", [(16, 1, 4096), (17, 1, 4096), (11, 3, 192), (13, 5, 4096), (37, 7, 320)])
+def test_step_fp32_projection_tiles(gpu, orc, S, T, ff):
+    """16 to 259 rows in one fp32 layer: each tile shape of the fp32 projections, with ragged last
+    tiles, K split in 4, 2 and 1, and K ranges shorter than the waves of a workgroup."""
+    cfg = gpu.EncoderConfig(layers=1, max_chunk=T, max_streams=S, dtype="f32", ff_dim=ff)
+    plan = lambda step, S, T: [T - (s % 4 == 1) for s in range(S)]
+    enc, _, _, res = _run_steps(gpu, orc, cfg, S=S, T=T, n_steps=1, seed=71 + S, seed_caches=True, valid_plan=plan)
+    for got, ref in res:
+        assert harness.rel_err(got, ref) <= 1e-4, (S, T, ff)
+    enc.close()

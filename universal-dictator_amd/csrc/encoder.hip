@@ -357,7 +357,7 @@ extern "C" UD_API int ud_encoder_create(const ud_encoder_config* cfg, ud_encoder
         ok &= (e->qkv = dev_alloc(R * 3 * D * esz)) != nullptr;
         ok &= (e->att = dev_alloc(Rp * D * esz)) != nullptr;
         ok &= (e->pw = (float*)dev_alloc(R * 2 * D * 4)) != nullptr;
-        if (e->bf) ok &= (e->part = (float*)dev_alloc(KSPLIT * R * D * 4)) != nullptr;
+        ok &= (e->part = (float*)dev_alloc(KSPLIT * R * D * 4)) != nullptr;
         ok &= (e->desc_dev = (int32_t*)dev_alloc(desc_ints(e) * 4)) != nullptr;
         if (ok) e->rows_dev = e->desc_dev + slots * DESC_INTS;
         ok &= (e->zero_row = dev_alloc(256)) != nullptr;
@@ -400,9 +400,17 @@ static int upload(void* dst, const void* src, size_t bytes) {
     return UD_OK;
 }
 
+// A `rows` x `cols` fp32 weight matrix (rows % 16 == 0, cols % 64 == 0) in the fp32 GEMM's layout.
+static int upload_frag_f32(float* dst, const float* src, size_t rows, size_t cols) {
+    std::vector<float> tmp(rows * cols);
+    const int nkb = (int)(cols / 16);
+    for (size_t r = 0; r < rows; r++)
+        for (size_t c = 0; c < cols; c += 4) memcpy(&tmp[frag_index_f32((int64_t)r, (int)c, nkb)], src + r * cols + c, 16);
+    return upload(dst, tmp.data(), tmp.size() * 4);
+}
+
 // Converts a `rows` x `cols` fp32 weight matrix to the encoder dtype and writes it at row offset
-// dst_row0 (a multiple of 16) of the destination: bf16 in the fragment-major GEMM layout, fp32
-// row-major.
+// dst_row0 (a multiple of 16) of the destination, in the GEMMs' fragment-major layouts.
 static int upload_matrix(ud_encoder* e, void* dst, size_t dst_row0, const float* src, size_t rows, size_t cols) {
     const size_t n = rows * cols;
     if (e->bf) {
@@ -417,7 +425,7 @@ static int upload_matrix(ud_encoder* e, void* dst, size_t dst_row0, const float*
                 tmp[frag_index((int64_t)r, (int)c, nk)] = host_weight16(src[r * cols + c], e->wf16);
         return upload(static_cast<uint16_t*>(dst) + dst_row0 * cols, tmp.data(), n * 2);
     }
-    return upload(static_cast<float*>(dst) + dst_row0 * cols, src, n * 4);
+    return upload_frag_f32(static_cast<float*>(dst) + dst_row0 * cols, src, rows, cols);
 }
 
 static bool parse_name(const char* name, int layers, int* layer, int* slot) {
@@ -439,7 +447,7 @@ static bool parse_name(const char* name, int layers, int* layer, int* slot) {
 // keeps conv.3 and conv.6 in fp32 -- WeightConverter.keepF32, Convert.swift:80 -- and rounds out
 // to f16; here the front-end's 1x1 convs run on the f16 MFMA as well.)
 static int upload_matrix_sub(ud_encoder* e, void* dst, const float* src, size_t rows, size_t cols) {
-    if (!e->bf) return upload(dst, src, rows * cols * 4);
+    if (!e->bf) return upload_frag_f32(static_cast<float*>(dst), src, rows, cols);
     const size_t n = rows * cols;
     for (size_t i = 0; i < n; i++)
         if (!(std::fabs(src[i]) <= kHalfMax))
@@ -594,12 +602,12 @@ extern "C" UD_API int ud_encoder_finalize(ud_encoder* e) {
     std::vector<uint16_t> Pb(e->bf ? pe.size() : 0);
     for (int li = 0; rc == UD_OK && li < e->layers; li++) {
         LayerDev& l = e->lw[li];
-        rc = upload(w_d, l.wpos.data(), (size_t)D * D * 4);
+        rc = upload_frag_f32(w_d, l.wpos.data(), D, D);
         if (rc != UD_OK) break;
         // P_l = PE . W_pos^T in fp32 (FastConformer.swift:168-174)
         GemmArgs g{};
         g.A = pe_d; g.W = w_d; g.C = p_d; g.M = n; g.N = D; g.K = D; g.lda = D; g.ldw = D; g.ldc = D;
-        g.epi = EPI_STORE_F32; g.act = 0; g.out_scale = 1.0f;
+        g.epi = EPI_STORE_F32; g.act = 0; g.out_scale = 1.0f; g.ksplit = 1;
         rc = launch_status(launch_gemm(g, false, nullptr), "position table");
         if (rc != UD_OK) break;
         if (e->bf) {
@@ -793,16 +801,16 @@ static Ws ws_view(ud_encoder* e, int s0, int T) {
     w.qkv = static_cast<char*>(e->qkv) + r0 * 3 * D * esz;
     w.att = static_cast<char*>(e->att) + r0 * D * esz;
     w.pw = e->pw + r0 * 2 * D;
-    w.part = e->part ? e->part + (size_t)KSPLIT * r0 * D : nullptr;
+    w.part = e->part + (size_t)KSPLIT * r0 * D;
     w.desc = e->desc_dev + (size_t)s0 * DESC_INTS;
     w.rows = e->rows_dev + r0;
     return w;
 }
 
 // encodeLayer (FastConformer.swift:262-321) for every layer, over streams s0 .. s0+n-1 of the step
-// (x and out point at their first row), on `st`.  The fp32 residual stream advances in place.  In
-// bf16 mode the residual projections write K-split partial slabs that the next LayerNorm folds into
-// the residual (in slab order); in fp32 mode they accumulate into it directly.
+// (x and out point at their first row), on `st`.  The fp32 residual stream advances in place: the
+// residual projections write K-split partial slabs that the next LayerNorm folds into the residual
+// (in slab order).
 static int enqueue_rows(ud_encoder* e, int s0, int n, int T, const float* x, float* out, hipStream_t st) {
     const int D = e->D, ff = e->ff, M = n * T;
     const bool bf = e->bf;
@@ -817,11 +825,10 @@ static int enqueue_rows(ud_encoder* e, int s0, int n, int T, const float* x, flo
     };
     // res += scale * A . W^T (N = D)
     auto resid = [&](const void* A, const void* W, int K, float scale, const char* what) -> int {
-        if (!bf) return gemm(A, W, w.res, D, K, D, EPI_RESID, ACT_NONE, scale, what);
         GemmArgs g{};
         g.A = A; g.W = W; g.C = w.part; g.M = M; g.N = D; g.K = K; g.lda = K; g.ldw = K; g.ldc = D;
         g.epi = EPI_PARTIAL; g.act = ACT_NONE; g.out_scale = scale;
-        g.ksplit = gemm_partial_splits(M, D, K);
+        g.ksplit = gemm_partial_splits(M, D, K, bf);
         pend.n = g.ksplit;
         return launch_status(launch_gemm(g, bf, st), what);
     };
@@ -1180,10 +1187,9 @@ static int launch_projection(ud_encoder* e, int which, int layer, int M, hipStre
         default:
             return fail(UD_ERR_INVALID, "ud_time_projection: projection %d", which);
     }
-    if (g.N == D) {                       // the residual projections: split-K slabs (16-bit) or +=
+    if (g.N == D) {                       // the residual projections: split-K slabs
         g.ldc = D;
-        if (e->bf) { g.C = e->part; g.epi = EPI_PARTIAL; g.ksplit = gemm_partial_splits(M, D, g.K); }
-        else { g.C = e->res; g.epi = EPI_RESID; }
+        g.C = e->part; g.epi = EPI_PARTIAL; g.ksplit = gemm_partial_splits(M, D, g.K, e->bf);
     }
     g.lda = g.K; g.ldw = g.K;
     if (flops) *flops = 2.0 * M * g.N * g.K;

@@ -18,7 +18,7 @@
 //    writes its own fp32 partial slab and the following LayerNorm adds the slabs, in order, to the
 //    residual row it reads anyway -- deterministic, no atomics, no extra kernel.
 // Epilogues: act + half store (row-major, or fragment-major for a following GEMM), fp32 store,
-// in-place fp32 residual accumulate, split-K partial slabs, and the QKV projection's split store:
+// split-K partial slabs, and the QKV projection's split store:
 // q row-major into the buffer the attention reads, K and V straight into their K/V ring rows (so
 // the new rows are written once, and the attention kernel only reads the rings).
 #include <type_traits>
@@ -487,56 +487,133 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_panel_kernel(Ge
     }
 }
 
-// ---------------------------------------------------------------- fp32 (VALU) GEMM
-// 64x64 tiles, 256 threads with 4x4 outputs each, K staged through LDS in slices of 16.
-constexpr int F_BM = 64, F_BN = 64, F_BK = 16;
+// ---------------------------------------------------------------- fp32 encoder (MFMA)
+// The fp32 encoder's projections and front-end on v_mfma_f32_16x16x4_f32, shaped as gemm_bf16_kernel:
+// a workgroup of 8 waves owns a 16*MT x 16*NT output tile and its waves take the 64-wide K chunks of
+// the workgroup's K split in turn; the 8 partial tiles are summed in LDS in wave order.  At few rows
+// the weights (92 MB a layer) bound it: they are stored fragment-major (frag_index_f32), so a wave
+// streams 4 KB of contiguous weights per chunk, and with one 16-column tile per workgroup and 2-4 K
+// splits of the N = 1024 projections 128-256 workgroups x 8 waves keep them in flight.  More rows
+// take wider tiles (launch_f32), which re-read the activations less often.
+// 8 rows: ff linear1 (4,096 x 1,024) 137 -> 5.9 us (2.8 TB/s), ff linear2 (1,024 x 4,096) 333 -> 5.9,
+// linear_out (1,024 x 1,024) 333 (its launches averaged with linear2's) -> 4.5; the 64 x 64 VALU
+// tiles before gave each CU at most one workgroup (16 for N = 1,024) that waited on every 16-wide K
+// slice in turn.  24-layer step: 4 streams x 2 frames 45.9 -> 1.75 ms.
+// Every output sums its K range in the same order whatever M is: a row's result does not depend on
+// the batch it is computed in.
+constexpr int F32_WK = 8;
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
-    __shared__ float As[F_BK][F_BM + 4];
-    __shared__ float Ws[F_BK][F_BN + 4];
+// Fragments of half a K chunk (32 columns): two 16 x 16 blocks per tile.
+template <int MT, int NT>
+struct Frag32 {
+    f32x4_t a[MT][2], b[NT][2];
+};
+
+template <int MT, int NT>
+__device__ __forceinline__ void mma_frag32(const Frag32<MT, NT>& f, f32x4_t (&acc)[NT][MT]) {
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.b[j][g][e], f.a[i][g][e], acc[j][i], 0, 0, 0);
+}
+
+template <int MT, int NT>
+__global__ __launch_bounds__(64 * F32_WK) void gemm_f32_kernel(GemmArgs a) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int nN = a.N / (16 * NT), nM = (a.M + 16 * MT - 1) / (16 * MT), ks = a.ksplit;
+    const int t = xcd_tile(blockIdx.x, nN * nM * ks);
+    const int kz = t % ks, tile = t / ks, nb = tile / nM, mb = tile % nM;
+    const int nk = a.K / 64, kper = nk / ks, kc0 = kz * kper;
     const float* A = static_cast<const float*>(a.A);
     const float* W = static_cast<const float*>(a.W);
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.y * F_BM, n0 = blockIdx.x * F_BN;
-    const int tm = (tid / 16) * 4, tn = (tid % 16) * 4;
-    // EPI_PARTIAL: blockIdx.z = K split kz over K range [kb, ke), its own fp32 slab.
-    const int kz = blockIdx.z;
-    const int kper = (a.K + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int kb = kz * kper, ke = min(a.K, kb + kper);
-    float acc[4][4] = {};
-    for (int k0 = kb; k0 < ke; k0 += F_BK) {
-        for (int idx = tid; idx < F_BM * F_BK; idx += 256) {
-            int r = idx / F_BK, kk = idx % F_BK;
-            int m = m0 + r, n = n0 + r, k = k0 + kk;
-            As[kk][r] = (m < a.M && k < ke) ? A[(int64_t)m * a.lda + k] : 0.0f;
-            Ws[kk][r] = (n < a.N && k < ke) ? W[(int64_t)n * a.ldw + k] : 0.0f;
+    // lane (r16, q): columns 4q .. 4q + 3 of row r16 of each 16 x 16 block; MFMA e takes element e of
+    // both operands, so they see the same permutation of a block's 16 k values.  Rows past M repeat
+    // the last one: computed, not stored.
+    const float* ap[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) ap[i] = A + (int64_t)min((mb * MT + i) * 16 + r16, a.M - 1) * a.lda + kc0 * 64 + 4 * q;
+    const float* wp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) wp[j] = W + ((int64_t)(nb * NT + j) * nk + kc0) * 1024 + lane * 4;
+    auto load = [&](Frag32<MT, NT>& f, int c, int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+#pragma unroll
+            for (int j = 0; j < NT; j++) f.b[j][g] = *reinterpret_cast<const f32x4_t*>(wp[j] + (int64_t)c * 1024 + (2 * h + g) * 256);
+#pragma unroll
+            for (int i = 0; i < MT; i++) f.a[i][g] = *reinterpret_cast<const f32x4_t*>(ap[i] + c * 64 + (2 * h + g) * 16);
         }
-        __syncthreads();
+    };
+    f32x4_t acc[NT][MT];
 #pragma unroll
-        for (int kk = 0; kk < F_BK; kk++) {
-            float av[4], wv[4];
+    for (int j = 0; j < NT; j++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) { av[i] = As[kk][tm + i]; wv[i] = Ws[kk][tn + i]; }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] += av[i] * wv[j];
-        }
-        __syncthreads();
+        for (int i = 0; i < MT; i++) acc[j][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    // chunks wave, wave + 8, ..; the next half chunk's loads are in flight behind this one's MFMAs
+    Frag32<MT, NT> f0, f1;
+    if (wave < kper) load(f0, wave, 0);
+    for (int c = wave; c < kper; c += F32_WK) {
+        load(f1, c, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_frag32<MT, NT>(f0, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + F32_WK < kper) load(f0, c + F32_WK, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_frag32<MT, NT>(f1, acc);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    for (int i = 0; i < 4; i++) {
-        int m = m0 + tm + i;
+    // acc[j][i] holds C^T: the lane's row is r16 of row tile i, its columns 4q .. 4q + 3 of tile j
+    __shared__ f32x4_t red[F32_WK][NT * MT][64];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) red[wave][j * MT + i][lane] = acc[j][i];
+    __syncthreads();
+    for (int idx = wave; idx < NT * MT; idx += F32_WK) {
+        const int j = idx / MT, i = idx % MT;
+        const int64_t m = (int64_t)(mb * MT + i) * 16 + r16;
+        const int n = (nb * NT + j) * 16 + 4 * q;
         if (m >= a.M) continue;
-        for (int j = 0; j < 4; j++) {
-            int n = n0 + tn + j;
-            if (n >= a.N) continue;
-            float* C = static_cast<float*>(a.C) + ((int64_t)kz * a.M + m) * a.ldc + n;
-            if (a.bias != nullptr && kz == 0) acc[i][j] += a.bias[n];
-            if (a.epi == EPI_RESID) *C = *C + a.out_scale * acc[i][j];
-            else if (a.epi == EPI_PARTIAL) *C = a.out_scale * acc[i][j];
-            else *C = apply_act(acc[i][j], a.act) * a.out_scale;
+        f32x4_t v = red[0][idx][lane];
+#pragma unroll
+        for (int w = 1; w < F32_WK; w++) v += red[w][idx][lane];
+        if (a.bias != nullptr) v += *reinterpret_cast<const f32x4_t*>(a.bias + n);
+        if (a.epi != EPI_PARTIAL) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = apply_act(v[e], a.act);
         }
+        *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.C) + ((int64_t)kz * a.M + m) * a.ldc + n) = v * a.out_scale;
     }
+}
+
+template <int MT, int NT>
+static int launch_f32_tile(const GemmArgs& a, hipStream_t st) {
+    const int tiles = a.N / (16 * NT) * ((a.M + 16 * MT - 1) / (16 * MT)) * a.ksplit;
+    hipLaunchKernelGGL((gemm_f32_kernel<MT, NT>), dim3(tiles), dim3(64 * F32_WK), 0, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// Row-major A, C and fragment-major W; EPI_STORE / EPI_STORE_F32 (with bias and activation) or
+// EPI_PARTIAL slabs.
+static int launch_f32(const GemmArgs& a, hipStream_t st) {
+    const bool partial = a.epi == EPI_PARTIAL;
+    if (!partial && a.epi != EPI_STORE && a.epi != EPI_STORE_F32) return -2;
+    if (partial && (a.bias != nullptr || a.act != ACT_NONE)) return -2;
+    if (a.N % 64 != 0 || a.K % 64 != 0 || a.lda % 4 != 0 || a.ldc % 4 != 0) return -2;
+    if (a.ksplit != (partial ? gemm_partial_splits(a.M, a.N, a.K, false) : 1)) return -2;
+    // 24-layer step, 16 x 7 rows: 64 x 64 tiles 5.4 ms, 64 x 32 4.0 (128 workgroups for ff linear1 become
+    // 256); 16 x 14: 6.1 and 6.2
+    if (a.M <= 16) return launch_f32_tile<1, 1>(a, st);
+    if (a.M <= 32) return launch_f32_tile<2, 1>(a, st);
+    if (a.M <= 64) return launch_f32_tile<4, 1>(a, st);
+    if (a.M <= 192) return launch_f32_tile<4, 2>(a, st);
+    return launch_f32_tile<4, 4>(a, st);
 }
 
 // ---------------------------------------------------------------- small-M fp32 (MFMA)
@@ -740,7 +817,11 @@ static Plan16 plan16(int M, int N, int K, int epi) {
     return best;
 }
 
-int gemm_partial_splits(int M, int N, int K) { return plan16(M, N, K, EPI_PARTIAL).ks; }
+int gemm_partial_splits(int M, int N, int K, bool half_data) {
+    if (half_data) return plan16(M, N, K, EPI_PARTIAL).ks;
+    // fp32: by K alone (see gemm_f32_kernel), at least a 64-wide chunk for each wave where it can be had
+    return K % 256 == 0 && K >= 2048 ? KSPLIT : K % 128 == 0 && K >= 1024 ? 2 : 1;
+}
 
 // Tile shapes measured on MI355X for the streaming step's M <= 128 projections (weights from HBM,
 // 48 rotating copies; the waves of a workgroup split K and share the reduction and the epilogue):
@@ -817,7 +898,7 @@ static int launch_half(const GemmArgs& a, hipStream_t st) {
         case EPI_QKV_RING: return launch_16<EPI_QKV_RING, ACT_NONE, false>(a, 1, st);
         case EPI_GLU: return launch_16<EPI_GLU, ACT_NONE, false>(a, 1, st);
         case EPI_PARTIAL: return a.act == ACT_NONE ? launch_16<EPI_PARTIAL, ACT_NONE, false>(a, a.ksplit, st) : -2;
-        default: return -2;   // the residual accumulate is an fp32-path epilogue
+        default: return -2;
     }
 }
 
@@ -834,14 +915,7 @@ int launch_gemm(const GemmArgs& a, bool half_data, hipStream_t st) {
             a.N != 3 * r.H * 128 || a.M % r.T != 0 || r.L + r.T > r.R || a.ldc < r.H * 128)
             return -2;
     }
-    if (!half_data) {
-        if (a.epi == EPI_STORE_FRAG) return -2;
-        const int ks = a.epi == EPI_PARTIAL ? a.ksplit : 1;
-        if (ks < 1 || ks > 64) return -2;
-        dim3 grid((a.N + F_BN - 1) / F_BN, (a.M + F_BM - 1) / F_BM, ks);
-        hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, st, a);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
+    if (!half_data) return launch_f32(a, st);
     if (a.K % 128 != 0) return -2;
     if (a.epi == EPI_SUBFLAT) {
         const SubFlat& f = a.flat;

@@ -82,10 +82,17 @@ __host__ __device__ inline int64_t frag_index(int64_t m, int c, int nk) {
     return (((int64_t)rt * nk + kc) << 10) + (h << 9) + ((g * 16 + r) << 3) + e;
 }
 
+// fp32 GEMM weights [N, K] (N % 16 == 0, K % 64 == 0) in the order the v_mfma_f32_16x16x4_f32 lanes
+// consume them: 1 KB blocks of 16 rows x 16 columns, element lane*4 + e (lane = 16*q + r) of block
+// (rt, kb) = W[16rt + r][16kb + 4q + e]; a row tile's blocks are contiguous along K.
+__host__ __device__ inline int64_t frag_index_f32(int64_t m, int c, int nkb) {
+    const int64_t rt = m >> 4;
+    return ((rt * nkb + (c >> 4)) << 8) + ((((c >> 2) & 3) * 16 + (m & 15)) << 2) + (c & 3);
+}
+
 // ---------------------------------------------------------------- GEMM  C = epi(A . W^T)
 enum Epi : int {
     EPI_STORE = 0,      // C[m,n] = act(acc) * out_scale, activation dtype, row-major
-    EPI_RESID = 1,      // C[m,n] += out_scale * acc   (C fp32 residual, in place)
     EPI_STORE_F32 = 3,  // C[m,n] = act(acc) * out_scale as fp32, row-major
     EPI_STORE_FRAG = 4, // as EPI_STORE but bf16 in fragment-major layout (the next GEMM's A)
     EPI_PARTIAL = 5,    // C[kz][m][n] = out_scale * (K-split kz partial), fp32; slabs M*ldc apart
@@ -120,7 +127,8 @@ struct QkvRing {
     int T, L, R, H;
 };
 // half_data: A [M, K] and W [N, K] IEEE half in fragment-major layout (lda/ldw unused); M may be any size, the
-// A buffer holding ceil(M/16)*16 rows.  fp32: row-major with leading dimensions lda/ldw/ldc.
+// A buffer holding ceil(M/16)*16 rows.  fp32: A and C row-major with leading dimensions lda/ldc, W
+// fragment-major (frag_index_f32).
 struct GemmArgs {
     const void* A; const void* W; void* C;
     int M, N, K, lda, ldw, ldc;
@@ -136,11 +144,11 @@ int launch_gemm(const GemmArgs& a, bool half_data, hipStream_t st);
 // [ks][M][ldc]) or EPI_STORE (ks = 1, optional bias, act).  K % (16 ks) == 0, lda and ldw multiples
 // of 4, A and W 16-byte aligned; any M and N.
 int launch_gemm_f32_small(const GemmArgs& a, int ks, hipStream_t st);
-// Most K splits of a 16-bit residual projection (partial slabs the workspace holds).
+// Most K splits of a residual projection (partial slabs the workspace holds).
 constexpr int KSPLIT = 4;
-// K splits (partial slabs) a 16-bit residual projection of this shape writes; launch_gemm expects it
-// in GemmArgs::ksplit for EPI_PARTIAL.
-int gemm_partial_splits(int M, int N, int K);
+// K splits (partial slabs) a residual projection of this shape writes; launch_gemm expects it in
+// GemmArgs::ksplit for EPI_PARTIAL.
+int gemm_partial_splits(int M, int N, int K, bool half_data);
 
 // ---------------------------------------------------------------- LayerNorm / conv / misc
 // Pending residual update: nparts fp32 slabs [rows, D] (stride rows*D) that a split-K residual
