@@ -121,3 +121,23 @@ def test_mel_error_paths(gpu):
     assert e.value.status == -2
     assert list(fe.features_device(2, a, 1000, [1000, 960], o, 7)) == [7, 7]
     fe.close()
+
+
+@pytest.mark.parametrize("n", [1, 45, 90])
+def test_frames_per_wave_and_wide_filterbank(gpu, orc, n):
+    """One, two and four frames per wave (the grid's size decides), with more bands than the band
+    sums' threads (200), bands wider than the weights a thread loads ahead, and a clip whose end cuts
+    its last frames' windows."""
+    ud = gpu
+    fb = np.zeros((200, 257), np.float32)
+    rng = np.random.default_rng(n)
+    for m in range(200):
+        lo = int(rng.integers(0, 250))
+        hi = min(257, lo + int(rng.integers(1, 40)))
+        fb[m, lo:hi] = rng.random(hi - lo, dtype=np.float32) * 0.02
+    win = refimpl.hann_symmetric()
+    clips = [harness.speechlike(16000 + 53 * b, 200 + b) for b in range(n)]
+    got = ud.MelFrontend(fb, win).features(clips)
+    ofe = orc.MelFrontend(fb, win)
+    for b in sorted({0, n // 2, n - 1}):
+        _close(got[b], ofe.features(clips[b]), "clip %d of %d" % (b, n))

@@ -221,8 +221,8 @@ struct MelJob {
 struct MelTables {
     const float* cos512; // cos(2 pi j / 512), j < 512
     const float* win;    // [400] analysis window
-    const float* fbT;    // [257][n_mels]
     const int2* krange;  // [n_mels] bins lo .. hi-1 hold band m's nonzero filterbank weights
+    const float* fbw;    // [widest band][n_mels]: weight of bin krange[m].x + j
     int n_mels;
 };
 int launch_mel(const MelTables& t, const MelJob* jobs_dev, int n_jobs, int max_nf, hipStream_t st);

@@ -3,28 +3,34 @@
 // The reference computes the features on the CPU (Sources/DictatorCore/Audio/NemoMel.swift:85-107):
 // two sgemms of the [T, 400] frame matrix against window-folded cos/sin tables [257, 400], the
 // power |X|^2 (as sqrt then square), a third sgemm against the filterbank and log(x + 2^-24).
-// Here one workgroup takes FR frames of one job (8, or 4 when the grid is small) and does all of
-// it in LDS:
+// Here a workgroup of 4 waves takes 4, 8 or 16 frames of one job; each wave transforms its own frames
+// and the workgroup sums the mel bands together:
 //
-//   stage    the frames' preemphasized samples times the window, sample-major (xs[n][t]), so one
-//            16-byte LDS read broadcasts 4 frames' sample n to the whole wave; the 512-entry
-//            cos table; all global loads of a thread are issued before its first LDS store
-//   DFT      thread k = bin k (0..255) runs over the 400 samples.  The angle of (k, n) is
-//            2 pi j / 512 with j = k (n + 56) mod 512 (the window sits at offset 56 of the
-//            512-point frame), so cos and -sin are two reads of the LDS cos table, at j and at
-//            j + 128; j advances by k per sample.  No global load in the loop: 2 table reads,
-//            FR / 4 broadcast frame reads and 2 * FR FMAs per sample.  Bin 256 (Nyquist) is a
-//            32-lane split reduction per frame
-//   power    into LDS pw[k][t]
-//   mel      thread (m, frame quad) sums fbT[k][m] * pw[k][t] over the bins from band m's first
-//            to its last nonzero weight (the products outside are +0, so the sum is the same as
-//            over all 257 bins for any finite power), then log
+//   frame    the 400 preemphasized, windowed samples, centred in 512 (offset 56), packed as 256
+//            complex values z[m] = x[2m] + i x[2m+1]; lane l loads m = l + 64 j, j < 4; the
+//            next frame's loads are in flight behind a frame's transform
+//   FFT      256 points, four radix-4 passes (decimation in frequency; Cooley and Tukey 1965) on four
+//            values per lane, with three exchanges through the wave's own LDS: no barrier
+//   split    X[k] of the real signal from Z[k] and Z[256 - k]: X = E - i W512^k O with
+//            E, O = (Z[k] +- conj Z[256 - k]) / 2 (O over i)
+//   power    |X|^2 into LDS (the reference takes the square root and squares it again)
+//   mel      thread (m, frame quad) sums w[m][k] * power[k][t] over the bins from band m's first to its
+//            last nonzero weight (the products outside are +0, so the sum is the same as over all 257
+//            bins for any finite power), then log.  A band's weights are stored from its first bin on,
+//            bin-major (fbw[j][m]), so the threads of a wave read neighbouring words
 //
-// Rounding: the reference multiplies x by float(cos) * window (its table entries); here
-// (x * window) * float(cos): the same terms to within an ulp each.  Every frame is computed the
-// same way wherever it sits in the grid and whatever FR (fixed summation order), so a frame
-// recomputed by a later streaming chunk is bit-identical to its first computation.  The preemphasis is evaluated as the
-// reference writes it, a[i] - 0.97 * a[i-1] with both roundings (contraction off).
+// 8 clips of 15-30 s (18,000 frames): 182 us a launch with the direct form (two 400-term sums per bin
+// against a cos table in LDS: 1.6 TFLOP/s of FMAs, where the transform needs a thirtieth of them),
+// 34.7 with flat sample loads and one range check per sample, 24.4 now; 24 clips of 19-37 s with their
+// call 544 -> 68.  What is left is VALU issue: about 300 instructions a frame for the transform and
+// the split, as many for the bands and the logarithm.
+//
+// Rounding: the reference multiplies x by float(cos) * window (its table entries) and sums 400 terms;
+// here x * window goes through the transform's 9 levels, whose rounding error is smaller.  Every frame
+// is computed the same way wherever it sits in the grid and however many frames its wave has (fixed
+// operation order), so a frame recomputed by a later streaming chunk is bit-identical to its first
+// computation.  The preemphasis is evaluated as the reference writes it, a[i] - 0.97 * a[i-1] with
+// both roundings (contraction off).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,127 +58,226 @@ __device__ __forceinline__ float preemph(float a, float prev) {
     return a - 0.97f * prev;
 }
 
-__device__ __forceinline__ float mel_power(float re, float im) {
-#pragma clang fp contract(off)
-    const float mag = sqrtf(re * re + im * im);
-    return mag * mag;
+typedef float __attribute__((address_space(1))) gfloat;   // global memory, for a pointer read from memory
+
+struct cpx {
+    float x, y;
+};
+__device__ __forceinline__ cpx operator+(cpx a, cpx b) { return {a.x + b.x, a.y + b.y}; }
+__device__ __forceinline__ cpx operator-(cpx a, cpx b) { return {a.x - b.x, a.y - b.y}; }
+// a (c - i s): a twiddle factor W = e^(-i angle) held as (cos, sin)
+__device__ __forceinline__ cpx twiddle(cpx a, cpx w) { return {a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y}; }
+
+// (cos, sin) of 2 pi j / 512 from the 512-entry cos table
+__device__ __forceinline__ cpx unit512(const float* cos512, int j) {
+    return {cos512[j & 511], cos512[(j + 384) & 511]};
 }
 
-template <int FR>
+// z[q] <- sum_j z[j] W4^(j q), then z[q] *= w[q - 1] for q > 0
+__device__ __forceinline__ void radix4(cpx (&z)[4], const cpx (&w)[3]) {
+    const cpx a = z[0] + z[2], b = z[0] - z[2], c = z[1] + z[3], d = z[1] - z[3];
+    z[0] = a + c;
+    z[1] = twiddle(cpx{b.x + d.y, b.y - d.x}, w[0]);
+    z[2] = twiddle(a - c, w[1]);
+    z[3] = twiddle(cpx{b.x - d.y, b.y + d.x}, w[2]);
+}
+
+// LDS slot of the transform's value i: the four bits above the low four permute those, so that every
+// pass reads and writes at most two lanes per bank
+__device__ __forceinline__ int fft_slot(int i) { return i ^ ((i >> 4) & 15); }
+
+// Orders a wave's LDS writes before its LDS reads of them (the wave's LDS operations run in order; this
+// keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int FPW>                                  // frames per wave
 __global__ __launch_bounds__(MEL_THREADS) void mel_kernel(const MelJob* __restrict__ jobs, MelTables tb) {
-    static_assert(FR == 4 || FR == 8, "frames per workgroup");
-    __shared__ float4 xs[MEL_WIN][FR / 4];
-    __shared__ float4 pw[MEL_NB][FR / 4];
-    __shared__ float cs[512];
+    static_assert(FPW == 1 || FPW == 2 || FPW == 4, "frames per wave");
+    constexpr int FR = 4 * FPW;                     // frames per workgroup
+    constexpr int QPT = FPW == 4 ? 2 : 1;           // frame quads per thread in the band sums
+    constexpr int MT = MEL_THREADS / (FPW / QPT);   // threads over the bands
+    constexpr int PRE = 8;                          // band weights a thread loads ahead
+    __shared__ float4 pw[FR / 4][MEL_NB];
+    __shared__ cpx ex[4][256];
     const MelJob J = jobs[blockIdx.y];
     const int j0 = blockIdx.x * FR;
     if (j0 >= J.nf) return;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nfr = min(FR, J.nf - j0);
     const long long fbase = J.f0 + j0;
 
-    constexpr int SU = (FR * MEL_WIN + MEL_THREADS - 1) / MEL_THREADS;
-    float* xsf = reinterpret_cast<float*>(xs);
-    float va[SU], vb[SU], wv[SU];
-    long long ix[SU];
+    // ---- the samples at 2m - 1, 2m, 2m + 1 of frame t's 512 (m = lane + 64 j).  Sample s of the frame
+    //      is clip sample base + s, base = 160 f - 256; a buffer over the part of the frame that the
+    //      clip (and the window's end) covers returns zeros for the rest.  (Buffer loads also count as
+    //      vector memory alone: flat ones, which these pointers would otherwise give, make every wait
+    //      for an LDS exchange wait for the next frame's samples too.)
+    struct Samples {
+        float v[4][3];
+        int end;                                    // the clip covers s < end
+        bool live;
+    };
+    auto load = [&](int t) __attribute__((always_inline)) {
+        Samples r;
+        const long long f = fbase + t, base = f * MEL_HOP - 256;
+        r.live = t < nfr && f < J.zero_from;
+        const int first = (int)min(max(J.first - base, 0ll), 1024ll);
+        r.end = r.live ? (int)min(max(J.n_audio - base, 0ll), 1024ll) : 0;
+        const int records = max(min(r.end, MEL_OFF + MEL_WIN) - first, 0);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(J.src + (base + first - J.first)), 0, records * 4, 0x00020000);
 #pragma unroll
-    for (int u = 0; u < SU; u++) {
-        const int e = tid + MEL_THREADS * u;
-        const int t = e / MEL_WIN, i = e - t * MEL_WIN;
-        const long long f = fbase + t;
-        ix[u] = -1;
-        va[u] = vb[u] = wv[u] = 0.0f;
-        if (e < FR * MEL_WIN && t < nfr && f < J.zero_from) {
-            const long long idx = f * MEL_HOP - 200 + i;
-            if (idx >= 0 && idx < J.n_audio) {
-                ix[u] = idx;
-                va[u] = J.src[idx - J.first];
-                if (idx > 0) vb[u] = J.src[idx - 1 - J.first];
-                wv[u] = tb.win[i];
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                // negative before the clip: beyond the buffer as an unsigned offset, if all of it is in
+                // the address register (the empty asm keeps an immediate from being split off, whose
+                // sum the range check would not wrap)
+                int off = (2 * (lane + 64 * j) - 1 + e - first) * 4;
+                asm volatile("" : "+v"(off));
+                r.v[j][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+            }
+        return r;
+    };
+    Samples cur = load(wave * FPW);
+
+    // ---- window weights; twiddle factors (of pass p, W_(4^(4 - p))^((lane's low index) q)); the
+    //      thread's band and its first weights
+    float wv[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = 2 * (lane + 64 * j) - MEL_OFF;
+        const bool in = i >= 0 && i < MEL_WIN;      // (the window's length is even)
+        wv[j][0] = in ? tb.win[i] : 0.0f;
+        wv[j][1] = in ? tb.win[i + 1] : 0.0f;
+    }
+    cpx w1[3], w2[3], w3[3], ws[4];
+#pragma unroll
+    for (int q = 1; q < 4; q++) {
+        w1[q - 1] = unit512(tb.cos512, 2 * lane * q);
+        w2[q - 1] = unit512(tb.cos512, 8 * (lane & 15) * q);
+        w3[q - 1] = unit512(tb.cos512, 32 * (lane & 3) * q);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) ws[j] = unit512(tb.cos512, lane + 64 * j);
+    const int band = tid % MT;
+    int2 kr = band < tb.n_mels ? tb.krange[band] : make_int2(0, 0);
+    float pre[PRE];
+#pragma unroll
+    for (int j = 0; j < PRE; j++) pre[j] = kr.x + j < kr.y ? tb.fbw[j * tb.n_mels + band] : 0.0f;
+
+    cpx* x = ex[wave];
+#pragma unroll
+    for (int u = 0; u < FPW; u++) {
+        const int t = wave * FPW + u;
+        float* pt = reinterpret_cast<float*>(pw[t / 4]) + t % 4;     // power of bin k at pt[4 k]
+        const Samples c = cur;
+        if (u + 1 < FPW) cur = load(t + 1);         // in flight behind this frame
+        if (!c.live) {                              // wave-uniform: a frame of zeros, or none
+#pragma unroll
+            for (int j = 0; j < 4; j++) pt[4 * (lane + 64 * j)] = 0.0f;
+            if (lane == 0) pt[4 * 256] = 0.0f;
+            continue;
+        }
+        cpx z[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            // (the clip's first sample is its own preemphasis: the one before it loads as 0)
+            z[j].x = preemph(c.v[j][1], c.v[j][0]) * wv[j][0];
+            z[j].y = preemph(c.v[j][2], c.v[j][1]) * wv[j][1];
+        }
+        if (lane < MEL_OFF / 2) z[0] = cpx{0.0f, 0.0f};              // outside the window
+        if (lane >= (MEL_OFF + MEL_WIN) / 2 - 192) z[3] = cpx{0.0f, 0.0f};
+        if (c.end < MEL_OFF + MEL_WIN) {            // wave-uniform: samples past the clip are zero padding
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int s = 2 * (lane + 64 * j);
+                if (s >= c.end) z[j].x = 0.0f;
+                if (s + 1 >= c.end) z[j].y = 0.0f;
             }
         }
-    }
-    const float c0 = tb.cos512[tid], c1 = tb.cos512[tid + MEL_THREADS];
+        // values of m = lane + 64 j -> digits q1 (stride 64 of the exchange), then q2, q3, q4
+        radix4(z, w1);
 #pragma unroll
-    for (int u = 0; u < SU; u++) {
-        const int e = tid + MEL_THREADS * u;
-        if (e < FR * MEL_WIN) {
-            const int t = e / MEL_WIN, i = e - t * MEL_WIN;
-            const float x = ix[u] < 0 ? 0.0f : ix[u] == 0 ? va[u] : preemph(va[u], vb[u]);
-            xsf[i * FR + t] = x * wv[u];
+        for (int q = 0; q < 4; q++) x[fft_slot(64 * q + lane)] = z[q];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; j++) z[j] = x[fft_slot((lane & 48) * 4 + (lane & 15) + 16 * j)];
+        wave_lds_fence();
+        radix4(z, w2);
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[fft_slot((lane & 48) * 4 + 16 * q + (lane & 15))] = z[q];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; j++) z[j] = x[fft_slot((lane & 60) * 4 + (lane & 3) + 4 * j)];
+        wave_lds_fence();
+        radix4(z, w3);
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[fft_slot((lane & 60) * 4 + 4 * q + (lane & 3))] = z[q];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; j++) z[j] = x[fft_slot(4 * lane + j)];
+        wave_lds_fence();
+        {
+            const cpx a = z[0] + z[2], b = z[0] - z[2], d = z[1] + z[3], e = z[1] - z[3];
+            z[0] = a + d;
+            z[1] = cpx{b.x + e.y, b.y - e.x};
+            z[2] = a - d;
+            z[3] = cpx{b.x - e.y, b.y + e.x};
         }
+        // lane = 16 q1 + 4 q2 + q3 holds Z[q1 + 4 q2 + 16 q3 + 64 q4]
+        const int k0 = (lane >> 4) + (lane & 12) + 16 * (lane & 3);
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[fft_slot(k0 + 64 * q)] = z[q];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = lane + 64 * j;
+            const cpx a = x[fft_slot(k)], b = x[fft_slot((256 - k) & 255)];
+            const cpx o = twiddle(cpx{0.5f * (a.x - b.x), 0.5f * (a.y + b.y)}, ws[j]);
+            const float re = 0.5f * (a.x + b.x) + o.y, im = 0.5f * (a.y - b.y) - o.x;
+            pt[4 * k] = re * re + im * im;
+            if (k == 0) pt[4 * 256] = (a.x - a.y) * (a.x - a.y);
+        }
+        wave_lds_fence();                           // the next frame's exchanges reuse x
     }
-    cs[tid] = c0;
-    cs[tid + MEL_THREADS] = c1;
     __syncthreads();
 
-    {
-        // bin 256: j = 256 (n + 56) mod 512; frame t = tid / 32 (< FR), lane l of 32 takes
-        // samples l, l + 32, ...; butterfly over the 32 lanes (xor offsets below 32 stay inside
-        // each half of the wave)
-        const int t = tid >> 5, l = tid & 31;
-        float r = 0.0f, q = 0.0f;
-        for (int n = l; t < FR && n < MEL_WIN; n += 32) {
-            const int j = (256 * (n + MEL_OFF)) & 511;
-            const float x = xsf[n * FR + t];
-            r = fmaf(cs[j], x, r);
-            q = fmaf(cs[(j + 128) & 511], x, q);
-        }
+    const int quad = tid / MT * QPT;                // frames 4 quad .. 4 (quad + QPT) - 1
+    gfloat* dst = (gfloat*)J.dst;
+    for (int m = band; m < tb.n_mels; m += MT) {
+        if (m != band) kr = tb.krange[m];
+        const float* w = tb.fbw + m;
+        float acc[QPT][4] = {};
+        auto add = [&](float fw, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int o = 16; o > 0; o >>= 1) {
-            r += __shfl_xor(r, o);
-            q += __shfl_xor(q, o);
-        }
-        if (l == 0 && t < FR) reinterpret_cast<float*>(pw[256])[t] = mel_power(r, q);
-    }
-    {
-        float re[FR], im[FR];
+            for (int h = 0; h < QPT; h++) {
+                const float4 p = pw[quad + h][k];
+                acc[h][0] = fmaf(fw, p.x, acc[h][0]);
+                acc[h][1] = fmaf(fw, p.y, acc[h][1]);
+                acc[h][2] = fmaf(fw, p.z, acc[h][2]);
+                acc[h][3] = fmaf(fw, p.w, acc[h][3]);
+            }
+        };
+        int k = kr.x;
+        if (m == band) {
 #pragma unroll
-        for (int t = 0; t < FR; t++) re[t] = im[t] = 0.0f;
-        const int k = tid;
-        int j = (k * MEL_OFF) & 511;
+            for (int j = 0; j < PRE; j++)
+                if (kr.x + j < kr.y) add(pre[j], kr.x + j);
+            k += PRE;
+        }
 #pragma unroll 4
-        for (int n = 0; n < MEL_WIN; n++) {
-            const float c = cs[j], s = cs[(j + 128) & 511];
-            j = (j + k) & 511;
+        for (; k < kr.y; k++) add(w[(k - kr.x) * tb.n_mels], k);
 #pragma unroll
-            for (int q = 0; q < FR / 4; q++) {
-                const float4 x = xs[n][q];
-                re[4 * q + 0] = fmaf(c, x.x, re[4 * q + 0]); im[4 * q + 0] = fmaf(s, x.x, im[4 * q + 0]);
-                re[4 * q + 1] = fmaf(c, x.y, re[4 * q + 1]); im[4 * q + 1] = fmaf(s, x.y, im[4 * q + 1]);
-                re[4 * q + 2] = fmaf(c, x.z, re[4 * q + 2]); im[4 * q + 2] = fmaf(s, x.z, im[4 * q + 2]);
-                re[4 * q + 3] = fmaf(c, x.w, re[4 * q + 3]); im[4 * q + 3] = fmaf(s, x.w, im[4 * q + 3]);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < FR / 4; q++)
-            pw[tid][q] = make_float4(mel_power(re[4 * q], im[4 * q]), mel_power(re[4 * q + 1], im[4 * q + 1]),
-                                     mel_power(re[4 * q + 2], im[4 * q + 2]), mel_power(re[4 * q + 3], im[4 * q + 3]));
-    }
-    __syncthreads();
-
-    constexpr int MT = MEL_THREADS / (FR / 4);   // threads per frame quad
-    const int quad = tid / MT;                    // frames 4 quad .. 4 quad + 3
-    for (int m = tid % MT; m < tb.n_mels; m += MT) {
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        const float* w = tb.fbT + m;
-        const int2 kr = tb.krange[m];
-#pragma unroll 8
-        for (int k = kr.x; k < kr.y; k++) {
-            const float fw = w[(long long)k * tb.n_mels];
-            const float4 p = pw[k][quad];
-            acc[0] = fmaf(fw, p.x, acc[0]);
-            acc[1] = fmaf(fw, p.y, acc[1]);
-            acc[2] = fmaf(fw, p.z, acc[2]);
-            acc[3] = fmaf(fw, p.w, acc[3]);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < 4 * QPT; i++) {
             const int t = 4 * quad + i;
-            if (t < nfr) {
-                const long long f = fbase + t;
-                J.dst[(long long)(j0 + t) * tb.n_mels + m] = f < J.zero_from ? logf(acc[i] + 5.9604644775390625e-8f) : 0.0f;
-            }
+            if (t < nfr)
+                dst[(long long)(j0 + t) * tb.n_mels + m] =
+                    fbase + t < J.zero_from ? logf(acc[i / 4][i % 4] + 5.9604644775390625e-8f) : 0.0f;
         }
     }
 }
@@ -180,11 +285,13 @@ __global__ __launch_bounds__(MEL_THREADS) void mel_kernel(const MelJob* __restri
 int launch_mel(const MelTables& t, const MelJob* jobs_dev, int n_jobs, int max_nf, hipStream_t st) {
     if (n_jobs < 1 || max_nf < 1) return 0;
     if (t.n_mels < 1 || t.n_mels > 256 || n_jobs > 65535) return -2;
-    // 8 frames per workgroup share each cos-table read; below 4 such workgroups per CU the
-    // grid is too small to hide the DFT loop's latency, and 4 frames per workgroup halve it
-    const int wg8 = (max_nf + 7) / 8 * n_jobs;
-    if (wg8 < 1024) mel_kernel<4><<<dim3((max_nf + 3) / 4, n_jobs), MEL_THREADS, 0, st>>>(jobs_dev, t);
-    else mel_kernel<8><<<dim3((max_nf + 7) / 8, n_jobs), MEL_THREADS, 0, st>>>(jobs_dev, t);
+    // The frames of a wave share its twiddle factors, its thread's band and the launch, and their loads
+    // run behind each other's transforms; with fewer than two workgroups per CU, fewer frames per wave
+    // fill more of the chip.
+    auto blocks = [&](int fr) { return (max_nf + fr - 1) / fr; };
+    if (blocks(16) * n_jobs >= 512) mel_kernel<4><<<dim3(blocks(16), n_jobs), MEL_THREADS, 0, st>>>(jobs_dev, t);
+    else if (blocks(8) * n_jobs >= 512) mel_kernel<2><<<dim3(blocks(8), n_jobs), MEL_THREADS, 0, st>>>(jobs_dev, t);
+    else mel_kernel<1><<<dim3(blocks(4), n_jobs), MEL_THREADS, 0, st>>>(jobs_dev, t);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -205,7 +312,7 @@ constexpr int MEL_RING = 4;   // job lists of ud_mel_features in flight before a
 
 struct ud_mel {
     int n_mels = 0;
-    float *cos512 = nullptr, *win = nullptr, *fbT = nullptr;
+    float *cos512 = nullptr, *win = nullptr, *fbw = nullptr;
     int2* krange = nullptr;
     // ring of job lists for ud_mel_features: slot i's pinned staging is rewritten only after the
     // kernel that read slot i's device copy has finished (its event)
@@ -216,13 +323,13 @@ struct ud_mel {
 };
 
 namespace ud {
-MelTables mel_tables_of(const ::ud_mel* m) { return MelTables{m->cos512, m->win, m->fbT, m->krange, m->n_mels}; }
+MelTables mel_tables_of(const ::ud_mel* m) { return MelTables{m->cos512, m->win, m->krange, m->fbw, m->n_mels}; }
 }  // namespace ud
 
 static void free_mel(ud_mel* m) {
     if (!m) return;
     (void)hipDeviceSynchronize();
-    for (void* p : {(void*)m->cos512, (void*)m->win, (void*)m->fbT, (void*)m->krange}) if (p) (void)hipFree(p);
+    for (void* p : {(void*)m->cos512, (void*)m->win, (void*)m->fbw, (void*)m->krange}) if (p) (void)hipFree(p);
     for (int i = 0; i < MEL_RING; i++) {
         if (m->djobs[i]) (void)hipFree(m->djobs[i]);
         if (m->hjobs[i]) (void)hipHostFree(m->hjobs[i]);
@@ -236,27 +343,30 @@ extern "C" UD_API int ud_mel_create(const float* fb_host, int32_t n_mels, const 
     *out = nullptr;
     if (n_mels < 1 || n_mels > 256) return mfail(UD_ERR_SHAPE, "ud_mel_create: n_mels %d outside 1..256", n_mels);
     // cos(2 pi j / 512) in double, rounded to float (the reference's float(cos(phase)),
-    // NemoMel.swift:33-35), the window as given, the filterbank transposed to [257][n_mels]
-    std::vector<float> cs(512), fbT((size_t)MEL_NB * n_mels);
+    // NemoMel.swift:33-35), the window as given, each band's filterbank weights from its first
+    // nonzero bin on, bin-major [widest band][n_mels]
+    std::vector<float> cs(512);
     for (int j = 0; j < 512; j++) cs[j] = (float)cos(2.0 * 3.14159265358979323846 * (double)j / 512.0);
     std::vector<int2> kr(n_mels);
+    int width = 1;
     for (int m = 0; m < n_mels; m++) {
         int lo = MEL_NB, hi = 0;
-        for (int k = 0; k < MEL_NB; k++) {
-            const float w = fb_host[(size_t)m * MEL_NB + k];
-            fbT[(size_t)k * n_mels + m] = w;
-            if (w != 0.0f) { lo = std::min(lo, k); hi = k + 1; }
-        }
+        for (int k = 0; k < MEL_NB; k++)
+            if (fb_host[(size_t)m * MEL_NB + k] != 0.0f) { lo = std::min(lo, k); hi = k + 1; }
         kr[m] = make_int2(lo < hi ? lo : 0, hi);
+        width = std::max(width, kr[m].y - kr[m].x);
     }
+    std::vector<float> fbw((size_t)width * n_mels);
+    for (int m = 0; m < n_mels; m++)
+        for (int k = kr[m].x; k < kr[m].y; k++) fbw[(size_t)(k - kr[m].x) * n_mels + m] = fb_host[(size_t)m * MEL_NB + k];
     ud_mel* m = new ud_mel();
     m->n_mels = n_mels;
     bool ok = hipMalloc(&m->cos512, 512 * 4) == hipSuccess && hipMalloc(&m->win, MEL_WIN * 4) == hipSuccess &&
-              hipMalloc(&m->fbT, fbT.size() * 4) == hipSuccess && hipMalloc(&m->krange, n_mels * sizeof(int2)) == hipSuccess;
+              hipMalloc(&m->fbw, fbw.size() * 4) == hipSuccess && hipMalloc(&m->krange, n_mels * sizeof(int2)) == hipSuccess;
     for (int i = 0; ok && i < MEL_RING; i++) ok = hipEventCreateWithFlags(&m->done[i], hipEventDisableTiming) == hipSuccess;
     ok = ok && hipMemcpy(m->cos512, cs.data(), 512 * 4, hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(m->win, window_host, MEL_WIN * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(m->fbT, fbT.data(), fbT.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(m->fbw, fbw.data(), fbw.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(m->krange, kr.data(), n_mels * sizeof(int2), hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) {
         free_mel(m);
