@@ -143,3 +143,34 @@ def test_offline_error_paths(gpu):
                                                        1, 4, 8, 128, 3, 7, None))
     with pytest.raises(ud.EngineError):
         ud.rel_pos_attention_batched(b, b, b, b, 3, b, b, b, b, 1, 4, 8, 7, head_dim=64)
+
+
+@pytest.mark.parametrize("B,Hh,T,left", [(1, 8, 1, None), (1, 2, 15, None), (1, 8, 33, None), (3, 2, 257, None),
+                                         (1, 8, 511, 70), (1, 1, 1500, 300), (3, 6, 257, None), (5, 8, 130, 40),
+                                         (1, 8, 513, 70)])
+def test_offline_query_block_kernels(gpu, orc, B, Hh, T, left):
+    """Up to 256 16-query blocks the waves of a workgroup split the keys, above it (the last three)
+    they share key tiles: fewer tiles than waves, several per wave, ragged last blocks and tiles,
+    per-query ranges, empty ranges and utterances of unequal length."""
+    ud = gpu
+    rng = np.random.default_rng(T + B)
+    D = Hh * DK
+    q, k, v = (ud.round_bf16(rng.standard_normal((B, T, D)).astype(np.float32)) for _ in range(3))
+    P = ud.round_bf16((rng.standard_normal((2 * T - 1, D)) * 0.5).astype(np.float32))
+    u, vb = ((rng.standard_normal((Hh, DK)) * 0.1).astype(np.float32) for _ in range(2))
+    i = np.arange(T)
+    ranges = np.zeros((B, T, 2), np.int32)
+    for b in range(B):
+        ranges[b, :, 0] = 0 if left is None else np.maximum(0, i // 14 * 14 - left)
+        ranges[b, :, 1] = np.minimum(T if left is None else i // 14 * 14 + 14, max(1, T - 7 * b))
+    if T > 1:
+        ranges[0, T // 2] = [5, 5]
+    dev = ud.DeviceBuffer.from_numpy
+    out = ud.DeviceBuffer(B * T * D * 2)
+    ud.rel_pos_attention_batched(dev(_bits(ud, q)), dev(_bits(ud, k)), dev(_bits(ud, v)), dev(_bits(ud, P)), T - 1,
+                                 dev(u), dev(vb), dev(ranges), out, B, T, Hh, P.shape[0])
+    ud.synchronize()
+    got = (out.download((B, T, D), np.uint16).astype(np.uint32) << 16).view(np.float32)
+    ref = np.stack([orc.relpos_attention(q[b], k[b], v[b], P, u, vb, ranges[b], T - 1, Hh) for b in range(B)])
+    assert T == 1 or not np.any(got[0, T // 2])
+    harness.assert_bf16_close(got, ref, "B=%d H=%d T=%d" % (B, Hh, T))

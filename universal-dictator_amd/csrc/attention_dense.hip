@@ -352,10 +352,230 @@ __global__ __launch_bounds__(512) void relpos_dense_kernel(DenseArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ few query blocks
+// One short utterance gives relpos_dense_kernel a grid far below the chip (30 s: 3 blocks of 128
+// queries x 8 heads = 24 workgroups), each of which sweeps every key tile in turn.  Here the keys are
+// what a workgroup's waves split: 8 waves own 16 queries of one (utterance, head), wave w takes the
+// 32-key tiles w, w + 8, .. of the block's key range with its own online softmax, and the 8 partial
+// results are merged once through LDS.  No tile is shared, so K and the band rows go straight from
+// global memory (L2) to registers as MFMA operands; V goes through the wave's own LDS for the
+// transposed reads, after the bd tile that the rel_shift gathers from has been read there.  A tile's
+// K and band registers are reloaded for the wave's next tile as soon as its products are issued.
+// The products, roundings and softmax are relpos_dense_kernel's; the price is that every 16 queries
+// read the keys again, hence the rule in launch_relpos_dense.
+// Per call, relpos_dense_kernel -> here, 8 heads: 1 x 40 frames 9.8 -> 5.5 us, 1 x 200 17.0 -> 9.4,
+// 1 x 377 (30 s) 23.4 -> 13.4, 8 x 60 11.5 -> 6.0.  Beyond the launch (2.5 us) it is bound by the L1
+// path of the operand rows: 28 KB per wave and tile.
+__global__ __launch_bounds__(512) void relpos_dense_few_kernel(DenseArgs a) {
+    using T = bf16;
+    constexpr int DK = 128, KT = 32, NW = 8, VST = DK + 16, SWS = 52;
+    // per wave: bd rows [16][SWS] floats, then V [KT][VST], at the end the partial output [8][64] float4
+    __shared__ __align__(16) char wl[NW][KT * VST * 2];
+    __shared__ float stat[NW][16][2];                 // per wave and query: exponent offset, sum
+    static_assert(16 * SWS * 4 <= KT * VST * 2 && 8 * 64 * 16 <= KT * VST * 2, "the regions overlay");
+
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int Tn = a.T, D = a.H * DK;
+    // heads fastest: consecutive workgroups read neighbouring columns of the same rows
+    const int nq = (Tn + 15) / 16, h = blockIdx.x % a.H, qb = blockIdx.x / a.H % nq, b = blockIdx.x / (a.H * nq);
+    const int iw = qb * 16;
+    const float c2 = a.scale * 1.4426950408889634f;
+    const T* Q = static_cast<const T*>(a.q) + (int64_t)b * Tn * D + h * DK;
+    const T* K = static_cast<const T*>(a.k) + (int64_t)b * Tn * D + h * DK;
+    const T* V = static_cast<const T*>(a.v) + (int64_t)b * Tn * D + h * DK;
+    const T* P = static_cast<const T*>(a.P) + h * DK;
+    const int32_t* R = a.ranges + (int64_t)b * Tn * 2;
+
+    // ---- the lane's query and its key range; the block's key tiles (union over its queries)
+    const int qi = iw + col;
+    const int qks = qi < Tn ? max(R[2 * qi], 0) : 0, qke = qi < Tn ? min(R[2 * qi + 1], Tn) : 0;
+    const bool any = qks < qke;
+    // (frame numbers below 2^24 are exact as floats)
+    const int lo = Tn - (int)group_max<16>(any ? (float)(Tn - qks) : 0.0f), hi = (int)group_max<16>(any ? (float)qke : 0.0f);
+    const int t_lo = __builtin_amdgcn_readfirstlane(lo) / KT;
+    const int t_hi = (__builtin_amdgcn_readfirstlane(hi) + KT - 1) / KT;
+
+    // ---- B operands: q + u, q + v in bf16 (query iw + col, k-chunk 4st + g)
+    uint4 aqu[4], aqv[4];
+    {
+        const T* qr = Q + (int64_t)min(qi, Tn - 1) * D;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            const int c = (4 * st + g) * 8;
+            float qf[8];
+            unpack16<T>(ld16(qr + c), qf);
+            uint32_t pu[4], pv[4];
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const float2 u = *reinterpret_cast<const float2*>(a.u + h * DK + c + e);
+                const float2 v = *reinterpret_cast<const float2*>(a.vb + h * DK + c + e);
+                pu[e / 2] = pack_bf16x2(qf[e] + u.x, qf[e + 1] + u.y);
+                pv[e / 2] = pack_bf16x2(qf[e] + v.x, qf[e + 1] + v.y);
+            }
+            aqu[st] = make_uint4(pu[0], pu[1], pu[2], pu[3]);
+            aqv[st] = make_uint4(pv[0], pv[1], pv[2], pv[3]);
+        }
+    }
+
+    // ---- a tile's operands: K rows 16ts + col, band rows rel = iw - j0 - 31 + 16tb + col, V rows
+    uint4 kf[2][4], pf[3][4], vf[8];
+    auto load_kp = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++) {
+            const T* r = K + (int64_t)min(t * KT + 16 * ts + col, Tn - 1) * D + g * 8;
+#pragma unroll
+            for (int st = 0; st < 4; st++) kf[ts][st] = ld16(r + 32 * st);
+        }
+#pragma unroll
+        for (int tb = 0; tb < 3; tb++) {
+            const int tr = min(max(iw - t * KT - (KT - 1) + 16 * tb + col + a.rel_offset, 0), a.n_rel - 1);
+            const T* r = P + (int64_t)tr * D + g * 8;
+#pragma unroll
+            for (int st = 0; st < 4; st++) pf[tb][st] = ld16(r + 32 * st);
+        }
+    };
+    auto load_v = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) vf[i] = ld16(V + (int64_t)min(t * KT + 4 * i + g, Tn - 1) * D + col * 8);
+    };
+    float* sw = reinterpret_cast<float*>(wl[wave]);
+    bf16* vl = reinterpret_cast<bf16*>(wl[wave]);
+
+    float m = -INFINITY;
+    f32x4_t lacc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, oacc[8];
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) oacc[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    int t = t_lo + wave;
+    if (t < t_hi) { load_kp(t); load_v(t); }
+    for (; t < t_hi; t += NW) {
+        const int j0 = t * KT;
+        const bool more = t + NW < t_hi;
+        // ---- ac = K . (q+u)^T, bd = P_band . (q+v)^T
+        f32x4_t sacc[2], bacc[3];
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++) sacc[ts] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int tb = 0; tb < 3; tb++) bacc[tb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+#pragma unroll
+            for (int ts = 0; ts < 2; ts++)
+                sacc[ts] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[ts][st]), as_bf16x8(aqu[st]), sacc[ts], 0, 0, 0);
+#pragma unroll
+            for (int tb = 0; tb < 3; tb++)
+                bacc[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(pf[tb][st]), as_bf16x8(aqv[st]), bacc[tb], 0, 0, 0);
+        }
+        if (more) load_kp(t + NW);
+#pragma unroll
+        for (int tb = 0; tb < 3; tb++)
+            *reinterpret_cast<float4*>(sw + col * SWS + 16 * tb + 4 * g) = make_float4(bacc[tb][0], bacc[tb][1], bacc[tb][2], bacc[tb][3]);
+        wave_lds_sync();
+        // ---- scores: key 16ts + 4g + r uses band row col - 16ts - 4g - r + 31 of the window
+        float sc[2][4];
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++) {
+            const float* bp = sw + col * SWS + col - 16 * ts - 4 * g + 28;
+#pragma unroll
+            for (int r = 0; r < 4; r++) sc[ts][r] = bp[3 - r];
+        }
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) sc[ts][r] += sacc[ts][r];
+        wave_lds_sync();                              // bd read: V takes its place
+#pragma unroll
+        for (int i = 0; i < 8; i++) *reinterpret_cast<uint4*>(vl + (4 * i + g) * VST + col * 8) = vf[i];
+        if (more) load_v(t + NW);
+        if (!__all(j0 >= qks && j0 + KT <= qke)) {    // keys outside a query's range: -inf
+#pragma unroll
+            for (int ts = 0; ts < 2; ts++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int j = j0 + 16 * ts + 4 * g + r;
+                    sc[ts][r] += (j >= qks && j < qke) ? 0.0f : -INFINITY;
+                }
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) mx = fmaxf(mx, sc[ts][r]);
+        mx = xmax32(xmax16(mx));
+        // the exponent offset is raised as in relpos_dense_kernel
+        const bool grow = (mx - m) * c2 > 8.0f;
+        if (__any(grow)) {
+            const float nm = grow ? mx : m;
+            const float corr = (m == -INFINITY || !grow) ? 1.0f : __builtin_amdgcn_exp2f((m - nm) * c2);
+            lacc *= corr;
+#pragma unroll
+            for (int dt = 0; dt < 8; dt++) oacc[dt] *= corr;
+            m = nm;
+        }
+        const float mc = m == -INFINITY ? 0.0f : m * c2;
+#pragma unroll
+        for (int ts = 0; ts < 2; ts++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) sc[ts][r] = __builtin_amdgcn_exp2f(fmaf(sc[ts][r], c2, -mc));
+        wave_lds_sync();
+        // ---- out^T += V^T . P^T over the tile's 32 keys (operand order as in relpos_dense_kernel)
+        const uint4 pb = make_uint4(pack_bf16x2(sc[0][0], sc[0][1]), pack_bf16x2(sc[0][2], sc[0][3]),
+                                    pack_bf16x2(sc[1][0], sc[1][1]), pack_bf16x2(sc[1][2], sc[1][3]));
+        const int k0 = 4 * g + (col >> 2);
+        lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u)),
+                                                      as_bf16x8(pb), lacc, 0, 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < 8; dt++) {
+            const int c0 = 16 * dt + 4 * (col & 3);
+            const v4i16_t b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16_t*)(vl + k0 * VST + c0));
+            const v4i16_t b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16_t*)(vl + (k0 + 16) * VST + c0));
+            uint4 av;
+            __builtin_memcpy(&av.x, &b0, 8);
+            __builtin_memcpy(&av.z, &b1, 8);
+            oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(av), as_bf16x8(pb), oacc[dt], 0, 0, 0);
+        }
+        wave_lds_sync();                              // V read: the next tile's bd may take its place
+    }
+
+    // ---- merge: wave w adds channels 16w .. 16w + 15 of the 8 partials, each rescaled from its own
+    //      exponent offset to the largest
+    f32x4_t* po = reinterpret_cast<f32x4_t*>(wl[wave]);
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) po[dt * 64 + lane] = oacc[dt];
+    if (g == 0) { stat[wave][col][0] = m; stat[wave][col][1] = lacc[0]; }
+    __syncthreads();
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; w++) M = fmaxf(M, stat[w][col][0]);
+    float l = 0.0f;
+    f32x4_t o = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float mw = stat[w][col][0];
+        const float f = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mw - M) * c2);
+        l += f * stat[w][col][1];
+        o += f * reinterpret_cast<const f32x4_t*>(wl[w])[wave * 64 + lane];
+    }
+    if (qi < Tn) {                                    // 0 for an empty key range
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        T* O = static_cast<T*>(a.out) + (int64_t)b * Tn * D + h * DK;
+        *reinterpret_cast<uint2*>(O + (int64_t)qi * D + 16 * wave + 4 * g) =
+            make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+    }
+}
+
 int launch_relpos_dense(const DenseArgs& a, hipStream_t st) {
     if (a.B < 1 || a.T < 1 || a.H < 1) return -2;
     const int64_t blocks = (int64_t)((a.T + 127) / 128) * a.H * a.B;
     if (blocks >= (1ll << 31)) return -2;
+    // One workgroup of the few-blocks kernel runs on a CU at a time, so it wins while its 16-query
+    // blocks fit the chip in one round: 256 blocks (1 x 500 frames x 8 heads) 27.5 -> 16.9 us, 384
+    // (2 x 377) 23.6 -> 25.6, 400 (1 x 800) 26.9 -> 30.3, 416 (4 x 200) 17.3 -> 17.8.
+    const int64_t few = (int64_t)((a.T + 15) / 16) * a.H * a.B;
+    if (few <= 256) {
+        hipLaunchKernelGGL(relpos_dense_few_kernel, dim3((unsigned)few), dim3(512), 0, st, a);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
     hipLaunchKernelGGL(relpos_dense_kernel, dim3((unsigned)blocks), dim3(512), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
