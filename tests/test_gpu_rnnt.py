@@ -192,3 +192,43 @@ def test_rnnt_error_paths(gpu):
     with pytest.raises(ud.EngineError) as e:
         ud.Rnnt(max_streams=2, hidden=96)            # hidden not a multiple of 64 (the GEMM tiles)
     assert e.value.status == -2
+
+
+@pytest.mark.parametrize("H,V,L,E", [(64, 33, 1, 16), (128, 70, 3, 48)])
+def test_small_decoders(gpu, orc, H, V, L, E):
+    """K ranges shorter than the waves of a workgroup, a vocabulary that ends inside a column tile, one
+    and three LSTM layers; projected rows at a 4-byte offset; 1 to 300 joint rows."""
+    ud = gpu
+    w = ud.synthetic_rnnt_weights(31, H=H, V=V, L=L, enc_dim=E, blank_bias=0.8)
+    r, ro = ud.Rnnt(max_streams=40, hidden=H, vocab=V, layers=L, enc_dim=E), orc.Rnnt(w)
+    r.set_weights(w)
+    rng = np.random.default_rng(32)
+    for n, frames in ((1, 1), (17, 2), (40, 8)):
+        for s in range(n):
+            r.reset(s)
+        f = rng.standard_normal((n, frames, H)).astype(np.float32)
+        buf = ud.DeviceBuffer.from_numpy(np.concatenate([np.zeros(1, np.float32), f.ravel()]))
+        buf.ptr += 4
+        got, cnt = r.greedy(list(range(n)), buf, frames, [frames] * n, cap=100)
+        buf.ptr -= 4
+        for b in range(n):
+            want = ro.greedy(f[b], ro.state())
+            assert cnt[b] == len(want) and got[b] == want, (n, b)
+    r.close()
+
+
+def test_projection_rows_independent_of_batch(gpu):
+    """A projected row has the same bits in every batch size (one to four row tiles, one and four column
+    tiles per workgroup)."""
+    ud = gpu
+    w = ud.synthetic_rnnt_weights(33)
+    r = ud.Rnnt(max_streams=1)
+    r.set_weights(w)
+    x = np.random.default_rng(34).standard_normal((300, 1024)).astype(np.float32)
+    xb, ob = ud.DeviceBuffer.from_numpy(x), ud.DeviceBuffer(300 * 640 * 4)
+    r.project(300, xb, ob)
+    full = ob.download((300, 640))
+    for rows in (1, 16, 17, 33, 64, 65, 256):
+        r.project(rows, xb, ob)
+        assert np.array_equal(ob.download((rows, 640)), full[:rows]), rows
+    r.close()

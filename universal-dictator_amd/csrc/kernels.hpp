@@ -140,10 +140,6 @@ struct GemmArgs {
     SubFlat flat;                   // EPI_SUBFLAT only
 };
 int launch_gemm(const GemmArgs& a, bool half_data, hipStream_t st);
-// fp32 GEMM for few rows (tens) on the fp32 MFMA: EPI_PARTIAL with ks K splits (slabs
-// [ks][M][ldc]) or EPI_STORE (ks = 1, optional bias, act).  K % (16 ks) == 0, lda and ldw multiples
-// of 4, A and W 16-byte aligned; any M and N.
-int launch_gemm_f32_small(const GemmArgs& a, int ks, hipStream_t st);
 // Most K splits of a residual projection (partial slabs the workspace holds).
 constexpr int KSPLIT = 4;
 // K splits (partial slabs) a residual projection of this shape writes; launch_gemm expects it in
