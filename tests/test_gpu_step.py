@@ -406,10 +406,10 @@ def test_recycled_slot_starts_clean_after_async_step(gpu, orc):
 
 
 
-@pytest.mark.parametrize("S,T", [(129, 1), (13, 11), (107, 3), (64, 11), (161, 7), (163, 11), (200, 14)])
+@pytest.mark.parametrize("S,T", [(1, 1), (17, 1), (11, 3), (65, 1), (9, 14), (129, 1), (13, 11), (107, 3), (64, 11), (161, 7), (163, 11), (200, 14)])
 def test_step_bf16_projection_tiles(gpu, orc, S, T):
-    """129 to 2,800 rows in one layer: each kernel that the 16-bit projections choose between (64 x 64
-    and 64 x 32 register tiles, 64 x 128, 128 x 128 and 112 x 256 row panels, one or several K splits), at row
+    """1 to 2,800 rows in one layer: each kernel that the 16-bit projections choose between (16 x 16 to
+    64 x 64 register tiles, 64 x 128, 128 x 128 and 112 x 256 row panels, one or several K splits), at row
     counts that leave a ragged last tile; some chunks partly valid."""
     cfg = gpu.EncoderConfig(layers=1, max_chunk=T, max_streams=S, dtype="bf16")
     plan = lambda step, S, T: [T - (s % 4 == 1) * min(T, 1 + s % 3) for s in range(S)]

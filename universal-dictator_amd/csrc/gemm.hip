@@ -710,35 +710,36 @@ int gemm_partial_splits(int M, int N, int K, bool half_data) {
     return K % 256 == 0 && K >= 2048 ? KSPLIT : K % 128 == 0 && K >= 1024 ? 2 : 1;
 }
 
-// Tile shapes measured on MI355X for the streaming step's M <= 128 projections (weights from HBM,
-// 48 rotating copies; the waves of a workgroup split K and share the reduction and the epilogue):
-//   ff linear1 (N 4096, K 1024, fragment out):  MT 2 x NT 4, 8 waves            6.97 -> 5.94 us
-//   q/k/v (N 3072, K 1024, half out):           MT 4 x NT 2, 8 waves            5.77 -> 5.53 us
-//   pointwise_conv1 (N 2048, K 1024, GLU out):  MT 2 x NT 2, 8 waves            4.31 -> 3.76 us
-//   ff linear2 (N 1024, K 4096, split-K 4):     MT 4 x NT 2, 8 waves            5.91 -> 5.76 us
-//   linear_out, pw2 (N 1024, K 1024):           MT 2 x NT 2, 8 waves, split-K 2 3.40 -> 3.12 us
-//                                               (half the slabs for the LayerNorm that adds them)
-//   subsampling out (N 1024, K 4352, bias):     MT 2 x NT 1, 8 waves: 256 workgroups of 8 or 9 chunks
-//                                               a wave (64 workgroups of 4 waves: ~4 us longer)
-// Wider tiles cut the re-reads of the activation panel; more waves per workgroup put more of a
-// tile's K range in flight at once.
+// At most 128 rows: the smallest tile (16 x 16, 16 x 32, 32 x 32, 64 x 32) that gives no CU a second
+// workgroup.  Such a launch streams its 2-8 MB of weights once, whatever the tile, so what counts is
+// that every CU has part of them in flight; a wider tile only cuts the re-reads of the activation
+// rows.  Four waves split K, eight where the K range is long (the subsampling's out: 4,352) and in the
+// tallest tile.  us per launch, weights from HBM, against the tiles tuned at 128 rows that all of these
+// had (32 x 64, 64 x 32, 32 x 32, all with 8 waves):
+//   rows                                    2             16            32            64            128
+//   ff linear1 (4,096 x 1,024)              6.1 -> 4.0    6.1 -> 4.0    6.1 -> 4.4    5.9 -> 4.8    5.8
+//   ff linear2 (1,024 x 4,096, 4 splits)    5.4 -> 3.8    5.4 -> 4.0    5.4 -> 4.3    5.4 -> 4.8    5.9
+//   q/k/v (3,072 x 1,024)                   5.7 -> 3.6    5.7 -> 3.7    5.7 -> 4.0    5.7 -> 4.5    5.5
+//   pointwise_conv1 (2,048 x 1,024, GLU)    4.0 -> 3.5    4.2 -> 3.9    4.4 -> 3.8    4.3 -> 3.8    4.3 -> 4.2
+//   linear_out (1,024 x 1,024, 2 splits)    2.9 -> 2.7    3.0 -> 2.7    3.0 -> 2.8    3.1 -> 3.0    3.4 -> 3.2
+//   subsampling out (1,024 x 4,352)         8.0 -> 7.2    8.4 -> 7.5    9.4 -> 7.2    9.0 -> 7.1    8.7
+template <int EPI, int ACT, bool BIAS, int MT, int NT>
+static int launch_few_tile(const GemmArgs& a, int ks, hipStream_t st) {
+    if (a.K / (64 * ks) >= 8 && (a.K / ks >= 2048 || MT == 4)) return launch_reg<MT, 8, NT, EPI, ACT, BIAS>(a, ks, st);
+    return launch_reg<MT, 4, NT, EPI, ACT, BIAS>(a, ks, st);
+}
 template <int EPI, int ACT, bool BIAS>
 static int launch_few(const GemmArgs& a, int ks, hipStream_t st) {
-    const bool k512 = a.K % (512 * ks) == 0;
-    if constexpr (BIAS) {
-        if (a.K >= 512) return launch_reg<2, 8, 1, EPI, ACT, true>(a, 1, st);
-        if (a.N % 32 == 0 && a.K % 256 == 0) return launch_reg<4, 4, 2, EPI, ACT, true>(a, 1, st);
-    } else if constexpr (EPI == EPI_STORE_FRAG) {
-        if (k512) return launch_reg<2, 8, 4, EPI, ACT>(a, 1, st);
-        return launch_reg<2, 2, 4, EPI, ACT>(a, 1, st);
-    } else if constexpr (EPI == EPI_STORE || EPI == EPI_QKV_RING) {
-        if (a.N % 32 == 0 && k512) return launch_reg<4, 8, 2, EPI, ACT>(a, 1, st);
-    } else if constexpr (EPI == EPI_STORE_F32 || EPI == EPI_GLU) {
-        if (a.N % 32 == 0 && k512) return launch_reg<2, 8, 2, EPI, ACT>(a, 1, st);
-    } else if constexpr (EPI == EPI_PARTIAL) {
-        if (a.N % 32 == 0 && k512)
-            return a.K >= 4096 ? launch_reg<4, 8, 2, EPI, ACT>(a, ks, st) : launch_reg<2, 8, 2, EPI, ACT>(a, ks, st);
-        if (a.K % (128 * ks) == 0) return launch_reg<4, 2, 1, EPI, ACT>(a, ks, st);
+    const int cus = device_cus();
+    auto fits = [&](int mt, int nt) { return a.N / (16 * nt) * ((a.M + 16 * mt - 1) / (16 * mt)) * ks <= cus; };
+    if (a.K / (64 * ks) >= 4) {
+        if constexpr (EPI != EPI_GLU)
+            if (fits(1, 1)) return launch_few_tile<EPI, ACT, BIAS, 1, 1>(a, ks, st);
+        if (a.N % 32 == 0) {
+            if (fits(1, 2)) return launch_few_tile<EPI, ACT, BIAS, 1, 2>(a, ks, st);
+            if (fits(2, 2)) return launch_few_tile<EPI, ACT, BIAS, 2, 2>(a, ks, st);
+            return launch_few_tile<EPI, ACT, BIAS, 4, 2>(a, ks, st);
+        }
     }
     return launch_reg<8, 2, EPI == EPI_GLU ? 2 : 1, EPI, ACT, BIAS>(a, ks, st);
 }
