@@ -220,3 +220,34 @@ def test_decode_error_paths(gpu):
         ud.gqa_attention_paged(b, b, b, b, 1 << 20, b, b, 1, 8, 2, 128, 65535 * 128 + 1, b)
     with pytest.raises(ud.EngineError):        # more than 65535 sequences (grid z)
         ud.gqa_attention_paged(b, b, b, b, 4, b, b, 65536, 8, 2, 128, 64, b)
+
+
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("Hq,Hkv,d,kv_dtype", [(32, 8, 128, "bf16"), (8, 8, 128, "bf16"), (16, 2, 64, "bf16"), (8, 4, 128, "f16")])
+@pytest.mark.parametrize("longest", [0, 1, 128, 129, 256])
+def test_single_split(gpu, orc, Hq, Hkv, d, kv_dtype, longest, M):
+    """Caches of one split, whose kernel writes the output itself: empty ranges of one query and of a
+    whole sequence give 0, windows."""
+    import test_gpu_decode_mq as mq
+    ud = gpu
+    rng = np.random.default_rng(longest + M + d)
+    lens = [longest, max(1, longest // 2), max(1, longest - 1), max(1, longest), max(1, longest)]
+    lens[0] = max(1, lens[0])
+    kseqs = [rng.standard_normal((L, Hkv * d)).astype(np.float32) for L in lens]
+    vseqs = [rng.standard_normal((L, Hkv * d)).astype(np.float32) for L in lens]
+    ranges = np.array([[[0, L if longest else 0]] * M for L in lens], np.int32)
+    ranges[1, :] = [0, 0]
+    ranges[2, M - 1] = [min(3, lens[2]), lens[2]] if longest else [0, 0]
+    ranges[3, 0] = [lens[3] // 2, lens[3] // 2]
+    q = rng.standard_normal((len(lens), M, Hq * d)).astype(np.float32)
+    pages = mq._pages(ud, kseqs, vseqs, Hkv, d, kv_dtype, rng)
+    got = mq.run_mq(ud, q, pages, ranges, Hq, Hkv, d, kv_dtype)
+    ref = mq.oracle_mq(orc, q, kseqs, vseqs, ranges, Hq, Hkv, kv_dtype)
+    assert not np.any(got[1]) and not np.any(got[3, 0])
+    if longest == 0:
+        assert not np.any(got)
+        return
+    if kv_dtype == "f16":
+        assert np.abs(got - ref).max() < 1e-4
+    else:
+        harness.assert_bf16_close(got[ranges[..., 0] < ranges[..., 1]], ref[ranges[..., 0] < ranges[..., 1]], "single split")

@@ -19,7 +19,8 @@
 //    v_permlane32_swap / v_permlane16_swap / DPP and across waves once through LDS;
 //  - bf16 pages at head_dim 128 take gqa_split_mfma_kernel instead: the same split with K staged
 //    in LDS by direct loads and both products on v_mfma_f32_16x16x32_bf16;
-//  - a second kernel merges the splits of each (sequence, head) with the usual max/sum rescaling.
+//  - a second kernel merges the splits of each (sequence, head) with the usual max/sum rescaling; a
+//    single split normalises and writes the output itself.
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -35,7 +36,6 @@ int ud_set_error(int code, const char* msg);   // encoder.hip
 namespace ud {
 
 constexpr int SPLIT = 128;      // keys per split workgroup (gqa_split_kernel)
-constexpr int MSPLIT = 256;     // keys per split workgroup of gqa_split_mfma_kernel (32 per wave)
 constexpr int PAGE = 16;        // block_size
 
 // Element formats of 16-bit K/V and RoPE rows (both stored as uint16_t).
@@ -125,6 +125,8 @@ struct GqaArgs {
     const int32_t* bt;
     const int32_t* ranges;         // [n][M][2]
     float* part;                   // [n][M][Hq][NS][D + 2]: unnormalised sum, max, sum of exp
+    float* out;                    // [n][M][Hq][D]; written by the split kernels when NS == 1 (a split
+                                   // is then a sequence's whole cache and no combine follows)
     int M;                         // queries per sequence (1 .. 8), all over the sequence's pages
     int max_blocks, Hq, Hkv, NS;
     int kmax;                      // keys the pages and the split grid can hold
@@ -147,7 +149,13 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     }
     const int s0 = split * SPLIT;
     const int ulo = max(lo, s0), uhi = min(hi, s0 + SPLIT);
-    if (ulo >= uhi) return;                       // this split holds no key of any query's range
+    const bool whole = a.NS == 1;
+    auto out_row = [&](int m, int gh) { return a.out + (((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * D; };
+    if (ulo >= uhi) {                             // this split holds no key of any query's range
+        if (whole)
+            for (int idx = tid; idx < M * G * D; idx += 256) out_row(idx / (G * D), idx / D % G)[idx % D] = 0.0f;
+        return;
+    }
     __shared__ float sc[G][SPLIT];
     __shared__ float stat[G][2];
     __shared__ __align__(16) float red[4][G][D];
@@ -186,7 +194,11 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     // turn (one read of the pages for all M queries).
     for (int qm = 0; qm < M; qm++) {
     const int klo = max(max(rg[2 * qm], 0), s0), khi = min(min(rg[2 * qm + 1], a.kmax), s0 + SPLIT);
-    if (klo >= khi) continue;                     // no key of this query's range here (uniform)
+    if (klo >= khi) {                             // no key of this query's range here (uniform)
+        if (whole)
+            for (int idx = tid; idx < G * D; idx += 256) out_row(qm, idx / D)[idx % D] = 0.0f;
+        continue;
+    }
     // ---- the G query heads of this kv head (8 channels per lane); for bf16 pages also as bf16
     //      pairs (channels 2e, 2e + 1) for the packed dot products
     float q[G][8];
@@ -324,6 +336,10 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     for (int idx = tid; idx < G * D; idx += 256) {
         const int g = idx / D, dd = idx % D;
         const float s = red[0][g][dd] + red[1][g][dd] + red[2][g][dd] + red[3][g][dd];
+        if (whole) {
+            out_row(qm, g)[dd] = s * (stat[g][1] > 0.0f ? 1.0f / stat[g][1] : 0.0f);
+            continue;
+        }
         float* pr = a.part + ((((int64_t)seq * M + qm) * a.Hq + kvh * G + g) * a.NS + split) * (D + 2);
         pr[dd] = s;
         if (dd == 0) { pr[D] = stat[g][0]; pr[D + 1] = stat[g][1]; }
@@ -334,12 +350,13 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
 
 // ---------------------------------------------------------------- bf16 pages, head_dim 128: MFMA
 // gqa_split_kernel's design with the products on the matrix cores and no K in registers:
-//  - 256-key splits, 8 waves of 32 keys (half the partials of 128-key splits);
-//  - one 64 KB LDS tile holds K, then V: K rows go global -> LDS with direct loads
+//  - KS-key splits of KS / 32 waves, 128 or 256 keys (launch_gqa's rule);
+//  - one KS x 256-byte LDS tile holds K, then V: K rows go global -> LDS with direct loads
 //    (global_load_lds_dwordx4) while V rows are loaded into registers; once every wave has read K,
 //    V (rows outside the range zeroed) is written over it.  Rows are 256 bytes, their 16-byte
 //    pieces permuted per row (kv_swz) by choosing each lane's source piece, so that the operand
-//    reads below fall on distinct banks.  About 68 KB of LDS: two workgroups per CU;
+//    reads below fall on distinct banks.  About 68 KB of LDS at 256 keys: two workgroups per CU, four
+//    at 128;
 //  - scores S^T = q . K^T on v_mfma_f32_16x16x32_bf16: A = q (rows = the G heads of the kv head,
 //    rounded once to bf16, zero rows above G), B = K^T (lane (c, g): key c, channels 8g .. 8g + 7),
 //    so lane (c, g) gets heads 4g .. 4g + 3 of key c;
@@ -367,9 +384,9 @@ __device__ __forceinline__ v4i16_t kv_tr16(const char* p) {
 // Query rows: the M queries of a sequence times the G query heads of the kv head, row r = m G + gh
 // (QR = M G rows, at most QM; RT = ceil(QM / 16) MFMA tiles of 16 rows).  Every K/V row of the
 // split is loaded once and multiplied against all of them.  QM == G is the one-query form.
-template <int G, int QM>
-__global__ __launch_bounds__(2 * MSPLIT) void gqa_split_mfma_kernel(GqaArgs a) {
-    constexpr int D = 128, ROWB = 2 * D, KS = MSPLIT, NWV = KS / 32;
+template <int G, int QM, int KS>
+__global__ __launch_bounds__(2 * KS) void gqa_split_mfma_kernel(GqaArgs a) {
+    constexpr int D = 128, ROWB = 2 * D, NWV = KS / 32;
     constexpr int DPW = (8 + NWV - 1) / NWV;      // channel tiles per wave (the last ones may have fewer)
     constexpr int RT = (QM + 15) / 16;
     constexpr bool ONE = QM == G;                 // one query per sequence
@@ -390,7 +407,13 @@ __global__ __launch_bounds__(2 * MSPLIT) void gqa_split_mfma_kernel(GqaArgs a) {
     }
     const int s0 = split * KS;
     const int klo = max(lo, s0), khi = min(hi, s0 + KS);
-    if (klo >= khi) return;                       // this split holds no key of any query's range
+    const bool whole = a.NS == 1;
+    if (klo >= khi) {                             // this split holds no key of any query's range
+        if (whole)
+            for (int idx = tid; idx < QR * D; idx += 2 * KS)
+                a.out[(((int64_t)seq * M + idx / (G * D)) * a.Hq + kvh * G + idx / D % G) * D + idx % D] = 0.0f;
+        return;
+    }
     constexpr int PROW = KS * 2 + 16;             // bytes per probability row (bf16, padded by 16 bytes)
     __shared__ __align__(16) char kv[KS * ROWB];         // K, then V
     __shared__ __align__(16) char pl[QM * PROW];         // probabilities, bf16 [row][key]
@@ -583,6 +606,20 @@ __global__ __launch_bounds__(2 * MSPLIT) void gqa_split_mfma_kernel(GqaArgs a) {
         const int row = 16 * rt + col;
         if (row < QR) {
             const int m = ONE ? 0 : row / G, gh = ONE ? row : row % G;
+            if (whole) {
+                float l = psum[0][row];
+#pragma unroll
+                for (int w = 1; w < NWV; w++) l += psum[w][row];
+                const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+                float* o = a.out + (((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * D + 4 * g;
+#pragma unroll
+                for (int u = 0; u < DPW; u++) {
+                    if (wave + NWV * u >= 8) break;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[16 * (wave + NWV * u) + e] = oacc[u][rt][e] * inv;
+                }
+                continue;
+            }
             float* pr = a.part + ((((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * a.NS + split) * (D + 2);
 #pragma unroll
             for (int u = 0; u < DPW; u++) {
@@ -738,46 +775,70 @@ extern "C" UD_API size_t ud_gqa_workspace_bytes(int32_t n, int32_t q_heads, int3
 
 // The MFMA split kernel for G query heads per kv head and M queries per sequence: QM query rows
 // (G for one query, else M G rounded up to whole 16-row tiles).
-template <int G>
-static int launch_mfma_g(const GqaArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+template <int G, int KS>
+static int launch_mfma_ks(const GqaArgs& a, dim3 grid, hipStream_t st) {
     const int rows = a.M * G;
-    if (a.M == 1) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, G>), grid, block, 0, st, a); return UD_OK; }
-    if (rows <= 16) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 16>), grid, block, 0, st, a); return UD_OK; }
+    const dim3 block(2 * KS);
+    if (a.M == 1) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, G, KS>), grid, block, 0, st, a); return UD_OK; }
+    if (rows <= 16) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 16, KS>), grid, block, 0, st, a); return UD_OK; }
     if constexpr (G >= 4) {
-        if (rows <= 32) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 32>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 32) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 32, KS>), grid, block, 0, st, a); return UD_OK; }
     }
     if constexpr (G == 8) {
-        if (rows <= 48) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 48>), grid, block, 0, st, a); return UD_OK; }
-        if (rows <= 64) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 64>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 48) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 48, KS>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 64) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 64, KS>), grid, block, 0, st, a); return UD_OK; }
     }
     return UD_ERR_SHAPE;
 }
+template <int G>
+static int launch_mfma_g(const GqaArgs& a, int split, dim3 grid, hipStream_t st) {
+    return split == 256 ? launch_mfma_ks<G, 256>(a, grid, st) : launch_mfma_ks<G, 128>(a, grid, st);
+}
+
+// Keys per split of the MFMA kernel.  128: twice the workgroups, four per CU, so that one's loads run
+// behind another's products; 256: half the partials.  us per call with pages from HBM, 256 -> 128, 8 kv
+// heads of 4 query heads: 1 x 1,000 keys 9.2 -> 8.2 (4 queries 10.8 -> 9.1), 24 sequences of 100-1,000
+// 21.9 -> 19.2, 8 of 512-4,096 23.7 -> 22.7, 16 of 512-4,096 37.7 -> 36.8 (4 queries 44.5 -> 44.9), 12 x 4
+// queries of 300-3,000 28.7 -> 27.8; 64 of 512-4,096 (8,192 splits of 256, pages partly in the last-level
+// cache) 122.1 -> 123.8, with 4 queries 144.5 -> 153.6.  A cache of 129-256 keys is one split of 256,
+// without a combine.
+static int mfma_split(int n, int kv_heads, int max_keys) {
+    if (max_keys <= 128) return 128;
+    const int64_t splits = (int64_t)n * kv_heads * ((max_keys + 255) / 256);
+    return max_keys <= 256 || splits >= 4096 ? 256 : 128;
+}
 
 // Grid of the split kernels: (kv head, split, sequence); the combine runs over the n M (sequence,
-// query) rows, whose ranges, partials and outputs are contiguous in that order.
+// query) rows, whose ranges, partials and outputs are contiguous in that order.  A single split writes
+// the output itself: 8 sequences of 60-120 keys 8.7 -> 5.1 us a call, 64 of 50-100 11.8 -> 6.2.
+template <int D>
+static void launch_combine(const GqaArgs& a, int n, int split, hipStream_t st) {
+    if (a.NS > 1)
+        hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.Hq, n * a.M), dim3(64), 0, st, a.part, a.ranges, a.out, a.Hq, a.NS,
+                           a.kmax, split);
+}
 template <typename KT, int D>
-static int launch_gqa(const GqaArgs& a, int n, int G, int nsplit, float* out, hipStream_t st) {
+static int launch_gqa(const GqaArgs& a, int n, int G, int split, hipStream_t st) {
     if constexpr (std::is_same<KT, BF16>::value && D == 128) {
         // bf16 pages at head_dim 128: the MFMA split kernel (grid as below)
-        dim3 grid(a.Hkv, nsplit, n), block(2 * MSPLIT);
+        dim3 grid(a.Hkv, a.NS, n);
         int rc;
         switch (G) {
-            case 1: rc = launch_mfma_g<1>(a, grid, block, st); break;
-            case 2: rc = launch_mfma_g<2>(a, grid, block, st); break;
-            case 4: rc = launch_mfma_g<4>(a, grid, block, st); break;
-            case 8: rc = launch_mfma_g<8>(a, grid, block, st); break;
+            case 1: rc = launch_mfma_g<1>(a, split, grid, st); break;
+            case 2: rc = launch_mfma_g<2>(a, split, grid, st); break;
+            case 4: rc = launch_mfma_g<4>(a, split, grid, st); break;
+            case 8: rc = launch_mfma_g<8>(a, split, grid, st); break;
             default: return UD_ERR_SHAPE;
         }
         if (rc != UD_OK) return rc;
-        hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.Hq, n * a.M), dim3(64), 0, st, a.part, a.ranges, out, a.Hq,
-                           a.NS, a.kmax, MSPLIT);
+        launch_combine<D>(a, n, split, st);
         return UD_OK;
     }
     // kv head fastest: the Hkv workgroups of one split run side by side and read each physical page's
     // Hkv x 4 KB as one contiguous block ([page][kv head][row][dim]); with the split fastest, the
     // workgroups in flight read scattered 4 KB pieces (measured on MI355X at 64 sequences, 8 kv
     // heads: 123.7 us per call against 143.8, and 106.0 against 113.1 for loads alone)
-    dim3 grid(a.Hkv, nsplit, n), block(256);
+    dim3 grid(a.Hkv, a.NS, n), block(256);
     switch (G) {
         case 1: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 1>), grid, block, 0, st, a); break;
         case 2: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 2>), grid, block, 0, st, a); break;
@@ -785,8 +846,7 @@ static int launch_gqa(const GqaArgs& a, int n, int G, int nsplit, float* out, hi
         case 8: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 8>), grid, block, 0, st, a); break;
         default: return UD_ERR_SHAPE;
     }
-    hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.Hq, n * a.M), dim3(64), 0, st, a.part, a.ranges, out, a.Hq, a.NS,
-                       a.kmax, SPLIT);
+    launch_combine<D>(a, n, SPLIT, st);
     return UD_OK;
 }
 
@@ -827,17 +887,18 @@ static int gqa_launch(const char* who, int32_t kv_dtype, const float* q_dev, con
     a.q = q_dev; a.kp = k_pages; a.vp = v_pages; a.bt = block_table; a.ranges = ranges_dev;
     a.part = workspace;
     a.M = n_queries;
-    // keys per split: MSPLIT on the MFMA path (bf16 pages, head_dim 128), SPLIT otherwise; the
-    // workspace is sized for SPLIT, the smaller, so it holds either
-    const int sp = kv_dtype == UD_BF16 && head_dim == 128 ? MSPLIT : SPLIT;
+    a.out = out_dev;
+    // keys per split: mfma_split on the MFMA path (bf16 pages, head_dim 128), SPLIT otherwise; the
+    // workspace is sized for SPLIT, the smallest, so it holds any
+    const int sp = kv_dtype == UD_BF16 && head_dim == 128 ? mfma_split(n, kv_heads, max_keys) : SPLIT;
     a.max_blocks = max_blocks; a.Hq = q_heads; a.Hkv = kv_heads; a.NS = nsplits(max_keys, sp);
     a.kmax = min(max_blocks * PAGE, a.NS * sp);
     a.scale = 1.0f / sqrtf((float)head_dim);
     int rc;
     if (kv_dtype == UD_BF16)
-        rc = head_dim == 128 ? launch_gqa<BF16, 128>(a, n, G, a.NS, out_dev, st) : launch_gqa<BF16, 64>(a, n, G, a.NS, out_dev, st);
+        rc = head_dim == 128 ? launch_gqa<BF16, 128>(a, n, G, sp, st) : launch_gqa<BF16, 64>(a, n, G, sp, st);
     else
-        rc = head_dim == 128 ? launch_gqa<F16, 128>(a, n, G, a.NS, out_dev, st) : launch_gqa<F16, 64>(a, n, G, a.NS, out_dev, st);
+        rc = head_dim == 128 ? launch_gqa<F16, 128>(a, n, G, sp, st) : launch_gqa<F16, 64>(a, n, G, sp, st);
     if (rc != UD_OK) return dfail(rc, "%s: unsupported shape", who);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return dfail(UD_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
