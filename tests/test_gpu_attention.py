@@ -112,6 +112,43 @@ def test_ring_attention_and_cache_update(gpu, orc, dtype, T, L):
     _ring_case(gpu, orc, dtype, T, L, 1.0)
 
 
+@pytest.mark.parametrize("n", [1, 3, 65, 129])
+def test_ring_attention_waves_per_workgroup(gpu, orc, n):
+    """The MFMA ring kernel with 2, 4 and 8 streams of a head per workgroup, the last workgroup partly
+    filled: three different streams against the oracle, and every stream that repeats one of them,
+    in whatever wave of whatever workgroup, bit-identical to it."""
+    ud, T, L, layer = gpu, 7, 70, 0
+    cfg = ud.EncoderConfig(layers=1, left_context=L, max_chunk=T, max_streams=n, dtype="bf16")
+    enc, model, _ = harness.make_encoder(ud, orc, cfg, seed=7)
+    D, H, m = cfg.d_model, cfg.heads, min(n, 3)
+    rng = np.random.default_rng(11)
+    streams = [enc.new_stream() for _ in range(n)]
+    st = harness.OracleState(m, cfg)
+    st.seed_random(rng, 0)
+    st.len[:] = [L, 33, 70][:m]
+    for i in range(0, n, m):
+        st.import_into(streams[i:i + m], ud, True)
+    valid = np.array([T, T - 2, 1], np.int32)[np.arange(n) % m]
+    qkv = ud.round_f16(rng.standard_normal((m, T, 3 * D)).astype(np.float32))
+    qbuf = _dev(ud, ud.f16_bits(qkv[np.arange(n) % m]))
+    att = ud.DeviceBuffer(n * T * D * 2)
+    enc.layer_attention(streams, T, layer, qbuf, att, valid=valid)
+    ud.synchronize()
+    bits = att.download((n, T, D), np.uint16)
+    P = ud.round_f16(model.P[layer])
+    for s in range(n):
+        if s >= m:
+            np.testing.assert_array_equal(bits[s], bits[s % m], err_msg="stream %d" % s)
+            continue
+        keys = np.concatenate([st.k[s, layer], qkv[s, :, D:2 * D]])
+        vals = np.concatenate([st.v[s, layer], qkv[s, :, 2 * D:]])
+        rr = np.array([[L - st.len[s], L + valid[s]]] * T, np.int32)
+        ref = orc.relpos_attention(qkv[s, :, :D], keys, vals, P, model.layers[layer][11], model.layers[layer][12], rr,
+                                   model.rel_offset, H)
+        harness.assert_bf16_close(ud.from_f16_bits(bits[s]), ref, "stream %d of %d" % (s, n))
+    enc.close()
+
+
 @pytest.mark.parametrize("T", [2, 14])
 def test_ring_attention_large_scores(gpu, orc, T):
     """q scaled by 8: scores with a spread of about +-25 before the softmax (a nearly one-hot

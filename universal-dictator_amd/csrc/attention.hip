@@ -836,9 +836,10 @@ int launch_ring_read_floor(const RingArgs& a, hipStream_t st) {
 // and the probabilities stay in registers as the B operand of P.V, whose k order is the same
 // permutation of the 32 rows of a piece: position 8g + e holds row 4g + e (e < 4), then
 // 16 + 4g + e - 4.  V is staged into LDS in that order.
-// One wave64 per (stream, head); a workgroup is 8 waves = 8 streams of one head, so the head's
-// band is loaded once per workgroup into LDS (it is the same for every stream), and every wave
-// is resident at once at two waves per SIMD (2,048 waves on 1,024 SIMDs).  Loads are spread over
+// One wave64 per (stream, head); a workgroup is NW waves = NW streams of one head, so the head's
+// band is loaded once per workgroup into LDS (it is the same for every stream), and at 256 streams
+// (NW = 8) every wave is resident at once at two waves per SIMD (2,048 waves on 1,024 SIMDs).  Fewer
+// streams take fewer waves per workgroup (launch_relpos_ring_mfma).  Loads are spread over
 // the unit so that the wave computes between them instead of stalling on issue: q and K first,
 // the first half of V after the band product, the second half after the key product.  When every
 // ring row is a valid key (ks = 0, ke = R: the steady state of full chunks) V needs no mask;
@@ -851,7 +852,6 @@ namespace rm {
 constexpr int BT = 7;                            // band tiles of 16 rows
 constexpr int BMAX = 16 * BT;
 constexpr int KMAX = 96;                         // ring rows (6 key tiles)
-constexpr int NW = 8;                            // waves (streams of one head) per workgroup
 constexpr int RS = 17;                           // 16-byte slots per band row in LDS (16 + 1 pad)
 constexpr int BSLOTS = BMAX * RS;                // 16-byte slots of the band rows
 constexpr int BINS = (BSLOTS + 64 + 63) / 64;     // direct-load instructions: band rows, u and v
@@ -886,8 +886,8 @@ __device__ __forceinline__ uint4 pack_f16x8_unit(const float (&x)[8]) {
 // KT key tiles cover ring rows 0 .. 16 KT - 1 (R <= 16 KT); NVL V loads cover rows 0 .. 4 NVL - 1.
 // NVL < 4 KT only when NVL == ceil(R / 4) (the launcher checks it), so that only the last V load
 // can reach past row R - 1.
-template <int KT, int NVL>
-__global__ __launch_bounds__(64 * rm::NW, 1) void relpos_ring_mfma_kernel(RingArgs a) {
+template <int KT, int NVL, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void relpos_ring_mfma_kernel(RingArgs a) {
     using namespace rm;
     using T = f16;
     constexpr int KP = (16 * KT + 31) / 32;       // 32-row V pieces
@@ -1148,23 +1148,39 @@ __global__ __launch_bounds__(64 * rm::NW, 1) void relpos_ring_mfma_kernel(RingAr
     }
 }
 
+template <int NW>
+static void launch_ring_mfma_waves(const RingArgs& a, hipStream_t st) {
+    const dim3 grid(a.H * ((a.n + NW - 1) / NW)), block(64 * NW);
+    const int kt = (a.R + 15) / 16, nvl = (a.R + 3) / 4;
+    if (kt == 6 && nvl == 21) hipLaunchKernelGGL((relpos_ring_mfma_kernel<6, 21, NW>), grid, block, 0, st, a);
+    else switch (kt) {
+        case 1: hipLaunchKernelGGL((relpos_ring_mfma_kernel<1, 4, NW>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((relpos_ring_mfma_kernel<2, 8, NW>), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((relpos_ring_mfma_kernel<3, 12, NW>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((relpos_ring_mfma_kernel<4, 16, NW>), grid, block, 0, st, a); break;
+        case 5: hipLaunchKernelGGL((relpos_ring_mfma_kernel<5, 20, NW>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((relpos_ring_mfma_kernel<6, 24, NW>), grid, block, 0, st, a); break;
+    }
+}
+
 int launch_relpos_ring_mfma(const RingArgs& a, hipStream_t st) {
     using namespace rm;
     if (a.T < 1 || a.T > 16 || a.R > KMAX || a.L + 2 * a.T - 1 > BMAX || a.n < 1 || a.H < 1 || !a.zero_row ||
         a.L + a.T > a.R)
         return -2;
     if (a.rel_offset + 1 - a.T < 0 || a.rel_offset + a.L + a.T - 1 >= a.n_rel) return -2;
-    const dim3 grid(a.H * ((a.n + NW - 1) / NW)), block(64 * NW);
-    const int kt = (a.R + 15) / 16, nvl = (a.R + 3) / 4;
-    if (kt == 6 && nvl == 21) hipLaunchKernelGGL((relpos_ring_mfma_kernel<6, 21>), grid, block, 0, st, a);
-    else switch (kt) {
-        case 1: hipLaunchKernelGGL((relpos_ring_mfma_kernel<1, 4>), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((relpos_ring_mfma_kernel<2, 8>), grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((relpos_ring_mfma_kernel<3, 12>), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((relpos_ring_mfma_kernel<4, 16>), grid, block, 0, st, a); break;
-        case 5: hipLaunchKernelGGL((relpos_ring_mfma_kernel<5, 20>), grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL((relpos_ring_mfma_kernel<6, 24>), grid, block, 0, st, a); break;
-    }
+    // The fewest of 2, 4 and 8 waves that give no CU a second workgroup: a launch of few units is one
+    // unit's chain of loads and products, which the other waves of its CU lengthen (LDS reads of the
+    // band, V through LDS), while more workgroups would load the band more often.  24-layer steps, us,
+    // 8 against 4 against 2 waves (1 wave is slower than 2 everywhere: 1,818 at 13 x 7):
+    //   streams x frames     13 x 7   16 x 14   64 x 7   96 x 7   128 x 14   200 x 7   256 x 14
+    //   8 waves              1,884    2,586     3,050    3,820    5,624      5,629     8,720
+    //   4 waves              1,811    2,485     2,981    3,745    5,590      5,717     8,790
+    //   2 waves              1,785    2,463     2,957    3,761    5,602      5,782     8,816
+    const int64_t units = (int64_t)a.H * a.n;
+    if (units <= 2 * 256) launch_ring_mfma_waves<2>(a, st);
+    else if (units <= 4 * 256) launch_ring_mfma_waves<4>(a, st);
+    else launch_ring_mfma_waves<8>(a, st);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
