@@ -149,6 +149,12 @@ def test_ring_attention_waves_per_workgroup(gpu, orc, n):
     enc.close()
 
 
+@pytest.mark.parametrize("T,L", [(2, 62), (2, 63), (4, 76), (8, 72), (8, 73)])
+def test_ring_attention_fp32_window_blocks(gpu, orc, T, L):
+    """fp32 windows of 64, 65, 80 and 81 keys: one block of 80 keys from 65 to 80, blocks of 64 around."""
+    _ring_case(gpu, orc, "f32", T, L, 1.0)
+
+
 @pytest.mark.parametrize("T", [2, 14])
 def test_ring_attention_large_scores(gpu, orc, T):
     """q scaled by 8: scores with a spread of about +-25 before the softmax (a nearly one-hot

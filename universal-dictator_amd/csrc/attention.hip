@@ -212,6 +212,7 @@ __device__ __forceinline__ void relpos_core(const Src& src, float scale) {
             if (idx < Tq * DK) {
                 int i = idx / DK, d = idx % DK;
                 float a = acc[o] * crow[i];
+#pragma unroll 8
                 for (int jj = 0; jj < nk; jj++) a += sc[i][jj] * to_f<T>(vs[jj][d]);
                 acc[o] = a;
             }
@@ -1237,6 +1238,17 @@ static int launch_ring_t(const RingArgs& a, hipStream_t st) {
     // 16-bit chunks of 5..16 frames (rings of R <= 96 rows): the MFMA kernel, one wave per (stream, head).
     if (sizeof(T) == 2 && a.T <= 16 && a.R <= 96 && a.L + 2 * a.T - 1 <= 112 && band_ok && a.zero_row)
         return launch_relpos_ring_mfma(a, st);
+    // fp32 windows of 65..80 keys and at most 8 frames: one block instead of 64 keys and a short second
+    // pass with its own loads and barriers (80 keys: 44-54 KB of LDS).  32 units of 72 keys, 2 frames:
+    // 11.7 -> 8.9 us a launch with P.V unrolled; 24-layer fp32 step 4 x 2 1,756 -> 1,700 us, 4 x 4
+    // 1,999 -> 1,908, 16 x 8 4,079 -> 3,922, 64 x 2 3,727 -> 3,683.
+    if constexpr (sizeof(T) == 4)
+        if (a.T <= 8 && a.L + a.T > 64 && a.L + a.T <= 80) {
+            if (a.T <= 2) hipLaunchKernelGGL((relpos_ring_kernel<T, 2, 80>), grid, block, 0, st, a);
+            else if (a.T <= 4) hipLaunchKernelGGL((relpos_ring_kernel<T, 4, 80>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((relpos_ring_kernel<T, 8, 80>), grid, block, 0, st, a);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
     if (a.T <= 2) hipLaunchKernelGGL((relpos_ring_kernel<T, 2, KeyBlock<T, 2>::KB>), grid, block, 0, st, a);
     else if (a.T <= 4) hipLaunchKernelGGL((relpos_ring_kernel<T, 4, KeyBlock<T, 4>::KB>), grid, block, 0, st, a);
     else if (a.T <= 8) hipLaunchKernelGGL((relpos_ring_kernel<T, 8, KeyBlock<T, 8>::KB>), grid, block, 0, st, a);
