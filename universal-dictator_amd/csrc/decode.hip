@@ -133,7 +133,10 @@ struct GqaArgs {
     float scale;
 };
 
-template <typename KT, int D, int G>
+// WHOLE: the only split of every sequence (NS == 1), which normalises and writes the output itself.  A
+// template parameter, of the MFMA kernel too: with both epilogues in one kernel, calls of several splits
+// took 0.3-2.8 % longer (1 x 4 queries, 500 keys, f16 and head_dim 64: 17.1 -> 17.5 us a call).
+template <typename KT, int D, int G, bool WHOLE>
 __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     constexpr int LPR = D / 8, RG = 256 / LPR, NP = SPLIT / RG, NV = G * 8;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -149,10 +152,9 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     }
     const int s0 = split * SPLIT;
     const int ulo = max(lo, s0), uhi = min(hi, s0 + SPLIT);
-    const bool whole = a.NS == 1;
     auto out_row = [&](int m, int gh) { return a.out + (((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * D; };
     if (ulo >= uhi) {                             // this split holds no key of any query's range
-        if (whole)
+        if constexpr (WHOLE)
             for (int idx = tid; idx < M * G * D; idx += 256) out_row(idx / (G * D), idx / D % G)[idx % D] = 0.0f;
         return;
     }
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     for (int qm = 0; qm < M; qm++) {
     const int klo = max(max(rg[2 * qm], 0), s0), khi = min(min(rg[2 * qm + 1], a.kmax), s0 + SPLIT);
     if (klo >= khi) {                             // no key of this query's range here (uniform)
-        if (whole)
+        if constexpr (WHOLE)
             for (int idx = tid; idx < G * D; idx += 256) out_row(qm, idx / D)[idx % D] = 0.0f;
         continue;
     }
@@ -336,13 +338,13 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     for (int idx = tid; idx < G * D; idx += 256) {
         const int g = idx / D, dd = idx % D;
         const float s = red[0][g][dd] + red[1][g][dd] + red[2][g][dd] + red[3][g][dd];
-        if (whole) {
+        if constexpr (WHOLE) {
             out_row(qm, g)[dd] = s * (stat[g][1] > 0.0f ? 1.0f / stat[g][1] : 0.0f);
-            continue;
+        } else {
+            float* pr = a.part + ((((int64_t)seq * M + qm) * a.Hq + kvh * G + g) * a.NS + split) * (D + 2);
+            pr[dd] = s;
+            if (dd == 0) { pr[D] = stat[g][0]; pr[D + 1] = stat[g][1]; }
         }
-        float* pr = a.part + ((((int64_t)seq * M + qm) * a.Hq + kvh * G + g) * a.NS + split) * (D + 2);
-        pr[dd] = s;
-        if (dd == 0) { pr[D] = stat[g][0]; pr[D + 1] = stat[g][1]; }
     }
     if (qm + 1 < M) __syncthreads();              // sc, stat and red are reused by the next query
     }
@@ -384,7 +386,7 @@ __device__ __forceinline__ v4i16_t kv_tr16(const char* p) {
 // Query rows: the M queries of a sequence times the G query heads of the kv head, row r = m G + gh
 // (QR = M G rows, at most QM; RT = ceil(QM / 16) MFMA tiles of 16 rows).  Every K/V row of the
 // split is loaded once and multiplied against all of them.  QM == G is the one-query form.
-template <int G, int QM, int KS>
+template <int G, int QM, int KS, bool WHOLE>
 __global__ __launch_bounds__(2 * KS) void gqa_split_mfma_kernel(GqaArgs a) {
     constexpr int D = 128, ROWB = 2 * D, NWV = KS / 32;
     constexpr int DPW = (8 + NWV - 1) / NWV;      // channel tiles per wave (the last ones may have fewer)
@@ -407,9 +409,8 @@ __global__ __launch_bounds__(2 * KS) void gqa_split_mfma_kernel(GqaArgs a) {
     }
     const int s0 = split * KS;
     const int klo = max(lo, s0), khi = min(hi, s0 + KS);
-    const bool whole = a.NS == 1;
     if (klo >= khi) {                             // this split holds no key of any query's range
-        if (whole)
+        if constexpr (WHOLE)
             for (int idx = tid; idx < QR * D; idx += 2 * KS)
                 a.out[(((int64_t)seq * M + idx / (G * D)) * a.Hq + kvh * G + idx / D % G) * D + idx % D] = 0.0f;
         return;
@@ -606,7 +607,7 @@ __global__ __launch_bounds__(2 * KS) void gqa_split_mfma_kernel(GqaArgs a) {
         const int row = 16 * rt + col;
         if (row < QR) {
             const int m = ONE ? 0 : row / G, gh = ONE ? row : row % G;
-            if (whole) {
+            if constexpr (WHOLE) {
                 float l = psum[0][row];
 #pragma unroll
                 for (int w = 1; w < NWV; w++) l += psum[w][row];
@@ -618,22 +619,22 @@ __global__ __launch_bounds__(2 * KS) void gqa_split_mfma_kernel(GqaArgs a) {
 #pragma unroll
                     for (int e = 0; e < 4; e++) o[16 * (wave + NWV * u) + e] = oacc[u][rt][e] * inv;
                 }
-                continue;
-            }
-            float* pr = a.part + ((((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * a.NS + split) * (D + 2);
+            } else {
+                float* pr = a.part + ((((int64_t)seq * M + m) * a.Hq + kvh * G + gh) * a.NS + split) * (D + 2);
 #pragma unroll
-            for (int u = 0; u < DPW; u++) {
-                if (wave + NWV * u >= 8) break;
-                float* o = pr + 16 * (wave + NWV * u) + 4 * g;
-                *reinterpret_cast<float2*>(o) = make_float2(oacc[u][rt][0], oacc[u][rt][1]);
-                *reinterpret_cast<float2*>(o + 2) = make_float2(oacc[u][rt][2], oacc[u][rt][3]);
-            }
-            if (wave == 0 && g == 0) {
-                float m = pmax[0][row], l = psum[0][row];
+                for (int u = 0; u < DPW; u++) {
+                    if (wave + NWV * u >= 8) break;
+                    float* o = pr + 16 * (wave + NWV * u) + 4 * g;
+                    *reinterpret_cast<float2*>(o) = make_float2(oacc[u][rt][0], oacc[u][rt][1]);
+                    *reinterpret_cast<float2*>(o + 2) = make_float2(oacc[u][rt][2], oacc[u][rt][3]);
+                }
+                if (wave == 0 && g == 0) {
+                    float m = pmax[0][row], l = psum[0][row];
 #pragma unroll
-                for (int w = 1; w < NWV; w++) { m = fmaxf(m, pmax[w][row]); l += psum[w][row]; }
-                pr[D] = m;
-                pr[D + 1] = l;
+                    for (int w = 1; w < NWV; w++) { m = fmaxf(m, pmax[w][row]); l += psum[w][row]; }
+                    pr[D] = m;
+                    pr[D + 1] = l;
+                }
             }
         }
     }
@@ -775,24 +776,25 @@ extern "C" UD_API size_t ud_gqa_workspace_bytes(int32_t n, int32_t q_heads, int3
 
 // The MFMA split kernel for G query heads per kv head and M queries per sequence: QM query rows
 // (G for one query, else M G rounded up to whole 16-row tiles).
-template <int G, int KS>
+template <int G, int KS, bool WHOLE>
 static int launch_mfma_ks(const GqaArgs& a, dim3 grid, hipStream_t st) {
     const int rows = a.M * G;
     const dim3 block(2 * KS);
-    if (a.M == 1) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, G, KS>), grid, block, 0, st, a); return UD_OK; }
-    if (rows <= 16) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 16, KS>), grid, block, 0, st, a); return UD_OK; }
+    if (a.M == 1) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, G, KS, WHOLE>), grid, block, 0, st, a); return UD_OK; }
+    if (rows <= 16) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 16, KS, WHOLE>), grid, block, 0, st, a); return UD_OK; }
     if constexpr (G >= 4) {
-        if (rows <= 32) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 32, KS>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 32) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 32, KS, WHOLE>), grid, block, 0, st, a); return UD_OK; }
     }
     if constexpr (G == 8) {
-        if (rows <= 48) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 48, KS>), grid, block, 0, st, a); return UD_OK; }
-        if (rows <= 64) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 64, KS>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 48) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 48, KS, WHOLE>), grid, block, 0, st, a); return UD_OK; }
+        if (rows <= 64) { hipLaunchKernelGGL((gqa_split_mfma_kernel<G, 64, KS, WHOLE>), grid, block, 0, st, a); return UD_OK; }
     }
     return UD_ERR_SHAPE;
 }
 template <int G>
 static int launch_mfma_g(const GqaArgs& a, int split, dim3 grid, hipStream_t st) {
-    return split == 256 ? launch_mfma_ks<G, 256>(a, grid, st) : launch_mfma_ks<G, 128>(a, grid, st);
+    if (a.NS == 1) return split == 256 ? launch_mfma_ks<G, 256, true>(a, grid, st) : launch_mfma_ks<G, 128, true>(a, grid, st);
+    return split == 256 ? launch_mfma_ks<G, 256, false>(a, grid, st) : launch_mfma_ks<G, 128, false>(a, grid, st);
 }
 
 // Keys per split of the MFMA kernel.  128: twice the workgroups, four per CU, so that one's loads run
@@ -817,6 +819,11 @@ static void launch_combine(const GqaArgs& a, int n, int split, hipStream_t st) {
         hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.Hq, n * a.M), dim3(64), 0, st, a.part, a.ranges, a.out, a.Hq, a.NS,
                            a.kmax, split);
 }
+template <typename KT, int D, int G>
+static void launch_split(const GqaArgs& a, dim3 grid, hipStream_t st) {
+    if (a.NS == 1) hipLaunchKernelGGL((gqa_split_kernel<KT, D, G, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gqa_split_kernel<KT, D, G, false>), grid, dim3(256), 0, st, a);
+}
 template <typename KT, int D>
 static int launch_gqa(const GqaArgs& a, int n, int G, int split, hipStream_t st) {
     if constexpr (std::is_same<KT, BF16>::value && D == 128) {
@@ -838,12 +845,12 @@ static int launch_gqa(const GqaArgs& a, int n, int G, int split, hipStream_t st)
     // Hkv x 4 KB as one contiguous block ([page][kv head][row][dim]); with the split fastest, the
     // workgroups in flight read scattered 4 KB pieces (measured on MI355X at 64 sequences, 8 kv
     // heads: 123.7 us per call against 143.8, and 106.0 against 113.1 for loads alone)
-    dim3 grid(a.Hkv, a.NS, n), block(256);
+    const dim3 grid(a.Hkv, a.NS, n);
     switch (G) {
-        case 1: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 1>), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 2>), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 4>), grid, block, 0, st, a); break;
-        case 8: hipLaunchKernelGGL((gqa_split_kernel<KT, D, 8>), grid, block, 0, st, a); break;
+        case 1: launch_split<KT, D, 1>(a, grid, st); break;
+        case 2: launch_split<KT, D, 2>(a, grid, st); break;
+        case 4: launch_split<KT, D, 4>(a, grid, st); break;
+        case 8: launch_split<KT, D, 8>(a, grid, st); break;
         default: return UD_ERR_SHAPE;
     }
     launch_combine<D>(a, n, SPLIT, st);
