@@ -251,3 +251,37 @@ def test_single_split(gpu, orc, Hq, Hkv, d, kv_dtype, longest, M):
         assert np.abs(got - ref).max() < 1e-4
     else:
         harness.assert_bf16_close(got[ranges[..., 0] < ranges[..., 1]], ref[ranges[..., 0] < ranges[..., 1]], "single split")
+
+
+@pytest.mark.parametrize("n,M,Hq,Hkv,max_keys,split", [
+    (1, 4, 32, 8, 300, 128), (8, 1, 8, 8, 4095, 128), (17, 1, 32, 8, 4096, 128), (18, 1, 32, 8, 4096, 256),
+    (31, 1, 8, 8, 2049, 128), (32, 1, 8, 8, 2049, 256), (52, 1, 32, 8, 2048, 128), (64, 1, 32, 8, 2048, 256),
+    (12, 4, 32, 8, 1024, 128), (13, 4, 32, 8, 1024, 256), (16, 3, 32, 8, 1000, 256), (16, 2, 64, 8, 1024, 256),
+    (17, 4, 32, 8, 1024, 128), (16, 2, 32, 8, 1024, 128), (9, 4, 32, 8, 4000, 128), (10, 4, 32, 8, 3841, 256),
+    (28, 4, 32, 8, 384, 128), (28, 4, 32, 8, 385, 256), (3, 1, 32, 8, 4096, 128), (4, 1, 32, 8, 4096, 256),
+    (24, 5, 32, 8, 4096, 128), (64, 8, 32, 8, 2048, 128)])
+def test_split_size_rule(gpu, orc, n, M, Hq, Hkv, max_keys, split):
+    """The keys per split follow the grid, the context and the query rows: read from the partials that a call
+    leaves in its workspace (every one written, none beyond).  All sequences share one page list."""
+    import test_gpu_decode_mq as mq
+    ud = gpu
+    d, blocks = 128, (max_keys + PAGE - 1) // PAGE
+    rng = np.random.default_rng(n + M + max_keys)
+    dev = ud.DeviceBuffer.from_numpy
+    k, v = (rng.standard_normal((max_keys, Hkv * d)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((n, M, Hq * d)).astype(np.float32)
+    kp, vp, table, max_blocks = mq._pages(ud, [k], [v], Hkv, d, "bf16", rng)
+    tables = dev(np.tile(table.download((1, max_blocks), np.int32), (n, 1)))
+    ends = max_keys - (M - 1) + np.arange(M)
+    ranges = np.tile(np.stack([np.zeros_like(ends), ends], -1)[None], (n, 1, 1)).astype(np.int32)
+    size = ud.gqa_workspace_bytes(n * M, Hq, d, max_keys)
+    qd, rd, ws, out = dev(q), dev(ranges), dev(np.full(size // 4, 0x7FC0DEAD, np.uint32)), ud.DeviceBuffer(q.nbytes)
+    ud.gqa_attention_paged_mq(qd, kp, vp, tables, max_blocks, rd, out, n, M, Hq, Hkv, d, max_keys, ws, kv_dtype="bf16")
+    ud.synchronize()
+    written = ws.download((size // 4,), np.uint32) != 0x7FC0DEAD
+    want = n * M * Hq * (d + 2) * -(-max_keys // split)
+    assert written.sum() == want and written[:want].all(), (written.sum() / want, split)
+    got = out.download(q.shape)
+    pick = [0, n - 1]
+    harness.assert_bf16_close(got[pick], mq.oracle_mq(orc, q[pick], [k, k], [v, v], ranges[pick], Hq, Hkv, "bf16"),
+                              "split of %d keys" % split)

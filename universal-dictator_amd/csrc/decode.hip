@@ -135,7 +135,7 @@ struct GqaArgs {
 
 // WHOLE: the only split of every sequence (NS == 1), which normalises and writes the output itself.  A
 // template parameter, of the MFMA kernel too: with both epilogues in one kernel, calls of several splits
-// took 0.3-2.8 % longer (1 x 4 queries, 500 keys, f16 and head_dim 64: 17.1 -> 17.5 us a call).
+// took 0.3-2.8 % longer (1 x 4 queries of 500 keys, 16/2 heads of 64: 17.1 -> 17.5 us a call).
 template <typename KT, int D, int G, bool WHOLE>
 __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
     constexpr int LPR = D / 8, RG = 256 / LPR, NP = SPLIT / RG, NV = G * 8;
@@ -797,17 +797,29 @@ static int launch_mfma_g(const GqaArgs& a, int split, dim3 grid, hipStream_t st)
     return split == 256 ? launch_mfma_ks<G, 256, false>(a, grid, st) : launch_mfma_ks<G, 128, false>(a, grid, st);
 }
 
-// Keys per split of the MFMA kernel.  128: twice the workgroups, four per CU, so that one's loads run
-// behind another's products; 256: half the partials.  us per call with pages from HBM, 256 -> 128, 8 kv
-// heads of 4 query heads: 1 x 1,000 keys 9.2 -> 8.2 (4 queries 10.8 -> 9.1), 24 sequences of 100-1,000
-// 21.9 -> 19.2, 8 of 512-4,096 23.7 -> 22.7, 16 of 512-4,096 37.7 -> 36.8 (4 queries 44.5 -> 44.9), 12 x 4
-// queries of 300-3,000 28.7 -> 27.8; 64 of 512-4,096 (8,192 splits of 256, pages partly in the last-level
-// cache) 122.1 -> 123.8, with 4 queries 144.5 -> 153.6.  A cache of 129-256 keys is one split of 256,
-// without a combine.
-static int mfma_split(int n, int kv_heads, int max_keys) {
+// Keys per split of the MFMA kernel, by the grid of 256-key splits, the longest context and the query rows
+// of a kv head.  128: twice the workgroups, four per CU instead of two, so that one's loads run behind
+// another's products and the last round costs less; 256: half the partials (520 bytes per query row and
+// split, for 64 KB of K and V in 128 keys).  A cache of 129-256 keys is one split of 256, without a combine.
+// us per call, 256 -> 128, 8 kv heads, pages from HBM, contexts from a quarter of the longest up:
+//   sequences x keys  1 x 1,000    24 x 1,000   8 x 4,000    32 x 2,000   24 x 4,000   64 x 4,000
+//   4 query rows      8.7 -> 7.9   19.2 -> 16.7 25.8 -> 24.3 40.0 -> 38.3 56.7 -> 56.7 135.8 -> 137.0
+//   16                10.3 -> 8.5  24.5 -> 22.8 30.4 -> 29.6 47.7 -> 47.4 66.3 -> 68.6 158.5 -> 168.4
+//   32                14.5 -> 11.3 45.2 -> 35.3 51.5 -> 39.7 94.0 -> 63.7 129 -> 89.3  321.6 -> 220.0
+// - Above 16 query rows a 256-key workgroup's tile and probabilities (83 KB) leave room for one per CU.
+// - Long contexts on a grid of several rounds gain nothing from smaller pieces, and pay for the partials.
+// - A grid of one and a half to two 256-key workgroups per CU is one round of them, nearly full: 16 x 1,000
+//   keys of equal contexts, 16 rows, 19.8 -> 21.5; 4 rows of 4,000 keys 17.1 -> 17.6.
+// What these lines leave: grids just below two or more whole rounds, all contexts equal, are 1-3 % slower in
+// 128-key splits at up to 8 rows and 4-6 % at 16; unequal contexts there are up to 18 % faster.
+static int mfma_split(int n, int kv_heads, int rows, int max_keys) {
     if (max_keys <= 128) return 128;
+    if (max_keys <= 256) return 256;
+    if (rows > 16) return 128;
     const int64_t splits = (int64_t)n * kv_heads * ((max_keys + 255) / 256);
-    return max_keys <= 256 || splits >= 4096 ? 256 : 128;
+    const bool many = splits >= 4096 || (max_keys > 2048 && splits >= (rows > 8 ? 1280 : 2304));
+    const bool one_round = splits > 384 && splits <= 512 && max_keys > (rows > 8 ? 384 : 2048);
+    return many || one_round ? 256 : 128;
 }
 
 // Grid of the split kernels: (kv head, split, sequence); the combine runs over the n M (sequence,
@@ -897,7 +909,7 @@ static int gqa_launch(const char* who, int32_t kv_dtype, const float* q_dev, con
     a.out = out_dev;
     // keys per split: mfma_split on the MFMA path (bf16 pages, head_dim 128), SPLIT otherwise; the
     // workspace is sized for SPLIT, the smallest, so it holds any
-    const int sp = kv_dtype == UD_BF16 && head_dim == 128 ? mfma_split(n, kv_heads, max_keys) : SPLIT;
+    const int sp = kv_dtype == UD_BF16 && head_dim == 128 ? mfma_split(n, kv_heads, n_queries * G, max_keys) : SPLIT;
     a.max_blocks = max_blocks; a.Hq = q_heads; a.Hkv = kv_heads; a.NS = nsplits(max_keys, sp);
     a.kmax = min(max_blocks * PAGE, a.NS * sp);
     a.scale = 1.0f / sqrtf((float)head_dim);
