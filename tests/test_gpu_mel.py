@@ -60,16 +60,18 @@ def test_frames_independent_of_batch(gpu, orc):
         assert np.array_equal(swapped[len(clips) - 1 - b], together[b])
 
 
-def test_frames_independent_of_workgroup_size(gpu, orc):
-    """A large call runs 8 frames per workgroup, a small one 4 (below 1024 workgroups of 8); a
-    clip's frames are bit-identical either way, and match the oracle in the large call."""
+@pytest.mark.parametrize("n", [45, 80])
+def test_frames_independent_of_workgroup_size(gpu, orc, n):
+    """A workgroup takes 16 frames (four per wave) in calls of at least 512 such workgroups (80 clips here),
+    else 8 (45 clips), else 4 (one clip); a clip's frames are bit-identical in all three, and match the oracle
+    in the large call."""
     ud = gpu
     fb, win = refimpl.slaney_mel_fb(), refimpl.hann_symmetric()
     fe = ud.MelFrontend(fb, win)
     ofe = orc.MelFrontend(fb, win)
-    clips = [harness.speechlike(16000 + 37 * b, 100 + b) for b in range(80)]   # 80 x 13 groups of 8
+    clips = [harness.speechlike(16000 + 37 * b, 100 + b) for b in range(n)]   # up to 111 or 119 frames
     big = fe.features(clips)
-    for b in (0, 41, 79):
+    for b in (0, n // 2 + 1, n - 1):
         alone = fe.features([clips[b]])[0]
         assert np.array_equal(alone.view(np.uint32), big[b].view(np.uint32)), b
         _close(big[b], ofe.features(clips[b]), "clip %d of the large call" % b)
