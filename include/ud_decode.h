@@ -45,7 +45,9 @@ extern "C" {
  * Precision: f16 pages are widened and used in fp32 arithmetic, as the reference kernel does.
  * bf16 pages use packed bf16 dot products: q and the softmax probabilities are rounded once to
  * bf16 (products exact, sums in fp32), within the bf16 activation bar (max abs 2e-2, cosine
- * 0.9995). */
+ * 0.9995).  Each split of the keys rounds its probabilities against its own maximum; at head_dim 128
+ * its size (128 or 256 keys) follows n, the query count, kv_heads and max_keys, so the last bits of a
+ * sequence's output may differ between calls that differ in these. */
 UD_API size_t ud_gqa_workspace_bytes(int32_t n, int32_t q_heads, int32_t head_dim, int32_t max_keys);
 UD_API int ud_gqa_attention_paged(int32_t kv_dtype, const float* q_dev, const void* k_pages, const void* v_pages,
                                   const int32_t* block_table, int32_t max_blocks, const int32_t* ranges_dev,

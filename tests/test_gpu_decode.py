@@ -117,8 +117,8 @@ def test_paged_gqa_ragged(gpu, orc, Hq, Hkv, d, kv_dtype):
 
 @pytest.mark.parametrize("d,kv_dtype", [(64, "bf16"), (64, "f16"), (128, "bf16")])
 def test_paged_gqa_long_context(gpu, orc, d, kv_dtype):
-    """Contexts past 64 splits (the combine merges them 64 at a time; 128-key splits, 256-key on the
-    MFMA path of bf16 pages at head_dim 128): 17,000 and 9,000 keys, a window [5,000, 13,100)
+    """Contexts past 64 splits (the combine merges them 64 at a time; splits of 128 keys at this grid,
+    test_split_size_rule has more than 64 of 256): 17,000 and 9,000 keys, a window [5,000, 13,100)
     whose first and last splits are partial, and a 300-key sequence in the same call."""
     ud = gpu
     rng = np.random.default_rng(61 + d)
@@ -259,7 +259,7 @@ def test_single_split(gpu, orc, Hq, Hkv, d, kv_dtype, longest, M):
     (12, 4, 32, 8, 1024, 128), (13, 4, 32, 8, 1024, 256), (16, 3, 32, 8, 1000, 256), (16, 2, 64, 8, 1024, 256),
     (17, 4, 32, 8, 1024, 128), (16, 2, 32, 8, 1024, 128), (9, 4, 32, 8, 4000, 128), (10, 4, 32, 8, 3841, 256),
     (28, 4, 32, 8, 384, 128), (28, 4, 32, 8, 385, 256), (3, 1, 32, 8, 4096, 128), (4, 1, 32, 8, 4096, 256),
-    (24, 5, 32, 8, 4096, 128), (64, 8, 32, 8, 2048, 128)])
+    (24, 5, 32, 8, 4096, 128), (64, 8, 32, 8, 2048, 128), (1, 1, 24, 6, 17000, 256)])
 def test_split_size_rule(gpu, orc, n, M, Hq, Hkv, max_keys, split):
     """The keys per split follow the grid, the context and the query rows: read from the partials that a call
     leaves in its workspace (every one written, none beyond).  All sequences share one page list."""
