@@ -364,7 +364,8 @@ __global__ __launch_bounds__(512) void relpos_dense_kernel(DenseArgs a) {
 // The products, roundings and softmax are relpos_dense_kernel's; the price is that every 16 queries
 // read the keys again, hence the rule in launch_relpos_dense.
 // Per call, relpos_dense_kernel -> here, 8 heads: 1 x 40 frames 9.8 -> 5.5 us, 1 x 200 17.0 -> 9.4,
-// 1 x 377 (30 s) 23.4 -> 13.4, 8 x 60 11.5 -> 6.0.  Beyond the launch (2.5 us) it is bound by the L1
+// 1 x 377 (30 s) 23.4 -> 13.4, 8 x 60 11.5 -> 6.0 (inputs in the last-level cache; 1 x 377 on inputs read for
+// the first time, with the wait for it, 39.9 -> 30.2).  Beyond the launch (2.5 us) it is bound by the L1
 // path of the operand rows: 28 KB per wave and tile.
 __global__ __launch_bounds__(512) void relpos_dense_few_kernel(DenseArgs a) {
     using T = bf16;

@@ -352,13 +352,13 @@ __global__ __launch_bounds__(256) void gqa_split_kernel(GqaArgs a) {
 
 // ---------------------------------------------------------------- bf16 pages, head_dim 128: MFMA
 // gqa_split_kernel's design with the products on the matrix cores and no K in registers:
-//  - KS-key splits of KS / 32 waves, 128 or 256 keys (launch_gqa's rule);
+//  - KS-key splits of KS / 32 waves, 128 or 256 keys (mfma_split);
 //  - one KS x 256-byte LDS tile holds K, then V: K rows go global -> LDS with direct loads
 //    (global_load_lds_dwordx4) while V rows are loaded into registers; once every wave has read K,
 //    V (rows outside the range zeroed) is written over it.  Rows are 256 bytes, their 16-byte
 //    pieces permuted per row (kv_swz) by choosing each lane's source piece, so that the operand
-//    reads below fall on distinct banks.  About 68 KB of LDS at 256 keys: two workgroups per CU, four
-//    at 128;
+//    reads below fall on distinct banks.  About 68 KB of LDS at 256 keys: two workgroups per CU (one
+//    above 16 query rows), four at 128;
 //  - scores S^T = q . K^T on v_mfma_f32_16x16x32_bf16: A = q (rows = the G heads of the kv head,
 //    rounded once to bf16, zero rows above G), B = K^T (lane (c, g): key c, channels 8g .. 8g + 7),
 //    so lane (c, g) gets heads 4g .. 4g + 3 of key c;

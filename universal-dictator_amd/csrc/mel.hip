@@ -22,15 +22,17 @@
 // 8 clips of 15-30 s (18,000 frames): 182 us a launch with the direct form (two 400-term sums per bin
 // against a cos table in LDS: 1.6 TFLOP/s of FMAs, where the transform needs a thirtieth of them),
 // 34.7 with flat sample loads and one range check per sample, 24.4 now; 24 clips of 19-37 s with their
-// call 544 -> 68.  What is left is VALU issue: about 300 instructions a frame for the transform and
-// the split, as many for the bands and the logarithm.
+// call 544 -> 68 (repeated calls: the samples come from the last-level cache; a first call on new samples,
+// with the wait for it, 191 -> 54 where a repeated one takes 164 -> 30).  What is left is VALU issue: about
+// 300 instructions a frame for the transform and the split, as many for the bands and the logarithm.
 //
 // Rounding: the reference multiplies x by float(cos) * window (its table entries) and sums 400 terms;
 // here x * window goes through the transform's 9 levels, whose rounding error is smaller.  Every frame
 // is computed the same way wherever it sits in the grid and however many frames its wave has (fixed
 // operation order), so a frame recomputed by a later streaming chunk is bit-identical to its first
 // computation.  The preemphasis is evaluated as the reference writes it, a[i] - 0.97 * a[i-1] with
-// both roundings (contraction off).
+// both roundings (contraction off); the transform and the power may use fused multiply-adds, alike in every
+// instantiation.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -19,7 +19,10 @@
 // through memory between launches.  An iteration is a chain of short kernels that the host waits for:
 // with the products split over workgroups it took nine (embedding, a product and a cell per layer, a
 // product, the joint's input, a product, the argmax) of 4-8 us each.
-// Now 6.0 us per LSTM layer (13 MB of weights, 2.2 TB/s), 3.3 joint.pred, 6.6 the joint of a few rows.
+// Now, up to 16 rows, 6.0 us per LSTM layer (13 MB of weights, 2.2 TB/s), 3.3 joint.pred, 6.6 the joint.
+// More rows cost more, since each of a product's workgroups (160 for a layer, 65 for the joint) reads all of
+// them: in a trace 6.3 us a layer up to 16 rows, 10.8 up to 32, 18.4 at 33-64 (0.7 TB/s of weights);
+// joint.pred 3.8, 5.2, 9.3; the joint 7.0, 9.5, 14.7.
 // A chunk of 2 frames that ends after 10 tokens: one stream 738 -> 373 us, 64 streams 911 -> 472;
 // 64 x 14 frames 1,826 -> 1,173.  joint.enc (rnnt_linear_kernel, one launch instead of slabs and their
 // sum): 128 rows 17.2 -> 12.2 us.
